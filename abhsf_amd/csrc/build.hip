@@ -384,7 +384,6 @@ SpmvLaunch Storage::launch() const
     SpmvLaunch L;
     L.bcol_bytes = bcol_bytes;
     L.val_bytes = val_bytes;
-    L.coo_single = nb[COO] > 0 && 4 * ne[COO] < 5 * nb[COO];  // mean entries per COO block below 1.25
     L.has_dense = nb[DENSE] > 0;
     L.bal.light = bal_light.get<uint32_t>();
     L.bal.pack = bal_pack.get<uint32_t>();
@@ -399,7 +398,7 @@ SpmvLaunch Storage::launch() const
     L.bal.n_slots = n_slots;
     L.bal.n_fix = n_fix;
     L.bal.tiled = tiled;
-    L.bal.tile_zs1 = tile_zs1;
+    L.bal.tile_sweep = tile_sweep;
     L.bal.coo_rng = bal_coo_rng.get<uint32_t>();
     return L;
 }
@@ -461,7 +460,7 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
     bal_order.release();
     bal_coo_rng.release();
     n_light = n_units = n_heavy = n_slots = n_fix = 0;
-    tile_zs1 = false;
+    tile_zs1 = tile_sweep = false;
     if (unit <= 0 || M == 0) return;
     ABHSF_REQUIRE(panels == 1 || panels == kXcdCount, ABHSF_ERR_INVALID, "column panels must match the XCD count");
     ABHSF_REQUIRE(tile_rows <= 0 || panels == 1, ABHSF_ERR_INVALID, "tiles and column panels do not combine");
@@ -645,11 +644,10 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
                 open_work = cw;
             }
         }
-        // blocks of 3 or more entries among the tiles' COO blocks (z - 1 >= 2):
-        // at one in 64 or more, most 64-block sub-chunks run phase B anyway
-        // and phase A takes one entry per block (R-MAT scale 22, s = 256:
-        // 9 % of them, 0.527 -> 0.51 ms; uniform scatter: none, and one entry
-        // per block would send the 0.15 % of blocks with two to phase B)
+        // Blocks of 3 or more entries among the tiles' COO blocks (z - 1 >= 2):
+        // below one in 64 the tiles are scattered, every gather a line of its
+        // own (uniform scatter: none; R-MAT scale 22: 9 %), and from n = 2^21
+        // on (x = 16 MB, four L2s) their sweep has to be kept together.
         uint64_t tile_blocks = 0, tile_ge3 = 0;
         for (const auto &it : items) {
             if (it.size() < 2) continue;
@@ -660,6 +658,7 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
                 }
         }
         tile_zs1 = tile_blocks > 0 && 64 * tile_ge3 >= tile_blocks;
+        tile_sweep = tile_blocks > 0 && !tile_zs1 && n > kSweepCols;
         // tiles first: they start together and sweep x in step (their COO
         // streams run in block-column order), the single strips fill the
         // remaining slots and follow

@@ -2,17 +2,19 @@
 //
 // One wavefront owns one strip (block row of s rows) and accumulates its
 // s x R output tile in LDS; the four scheme groups of the strip are walked in
-// turn (COO, CSR, bitmap, dense), each with a decode specialised to its layout:
-//   COO / CSR  element-parallel: E = 64/R entries per wave step, R right-hand
-//              sides per entry; the entry's block is found by a binary search
-//              over a 64-block chunk's inclusive nnz prefix (wave scan in LDS);
-//              CSR rows come from a binary search over the block's row pointers.
-//   bitmap     position-parallel: lane i of a 64-bit word tests bit i, the value
-//              offset is popcount(word & lanemask_lt) (the word is wave-uniform);
-//   dense      the bitmap walk with every bit set.
-// Products of the same output row are summed with xor-shuffles inside the wave
-// where rows are known to be contiguous (bitmap, dense) and with LDS atomic
-// adds where they are not (COO, CSR).
+// turn (COO, CSR, bitmap, dense), each with a decode specialised to its layout.
+// One right-hand side:
+//   COO / CSR  entry-parallel in storage order, 64 consecutive entries per
+//              load; an entry's block (COO) or block row (CSR) is the number of
+//              segment ends before it in a bit mask in LDS;
+//   bitmap     a lane owns consecutive positions and walks their set bits;
+//   dense      16- and 32-row blocks in 1 KB wave steps, else as bitmap.
+// Several right-hand sides: COO and bitmap windows of 64 entries decoded into
+// LDS (block by binary search over the chunk's prefix sums), CSR rows by lane,
+// dense blocks on the FP64 matrix cores where the tile is wide enough.
+// Products of the same output row are summed in registers and DPP where rows
+// are known to be contiguous (bitmap, dense) and with LDS atomic adds where
+// they are not.
 //
 // Reference semantics: y[lrow] += v * x[bcol*s + lcol] per scheme
 // (spmv/orig/88.cpp:214-235 COO, 88_bitmap.cpp:183-207 bitmap, 88.cpp:587-604
@@ -32,6 +34,43 @@
 
 namespace abhsf {
 namespace {
+
+// The single-RHS kernels read the matrix descriptor through the constant
+// address space, field by field where a group needs it (scalar loads), and
+// each group starts from a pointer and a lane number the compiler cannot see
+// through.  With the descriptor passed by value the compiler kept fields and
+// lane addresses of all four groups for the whole kernel: 83 VGPRs and 57
+// spilled SGPRs where the same groups now take 61 and 3.
+using MatPtr = const __attribute__((address_space(4))) DevMat *;
+using BalPtr = const __attribute__((address_space(4))) Balance *;
+
+template <typename P>
+__device__ inline P opaque_s(P p)
+{
+    const uint64_t v = (uint64_t)p;
+    uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    asm volatile("" : "+s"(lo), "+s"(hi));
+    return (P)(((uint64_t)hi << 32) | lo);
+}
+__device__ inline int opaque_v(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// A pointer read from a descriptor, known to point to device memory (global
+// instead of flat loads).
+template <typename T>
+__device__ inline const T *glob(const void *p)
+{
+    return (const T *)(const __attribute__((address_space(1))) T *)p;
+}
+template <typename T>
+__device__ inline T *glob_rw(T *p)
+{
+    return (T *)(__attribute__((address_space(1))) T *)p;
+}
 
 template <typename T>
 __device__ inline T ld(const void *p, uint64_t i) { return static_cast<const T *>(p)[i]; }
@@ -121,194 +160,276 @@ __device__ inline void group_reduce(int P, double &hi, double &lo)
     }
 }
 
-// CSR group, blocks [b0, b1) whose first value is at offset e.  Lanes own
-// block rows: for s <= 64 a wave step covers 64/s blocks (lane l -> block l/s,
-// row l%s), for s > 64 one block in s/64 row passes.  A lane reads its row's
-// bounds from the block's row pointers, sums the row's products in registers
-// and adds the sum to the strip accumulator: no search, one LDS update per
-// row.  s_st holds the chunk's exclusive value offsets, s_bc its block columns.
-template <typename VT, typename BT, typename RT, bool COMP>
-__device__ inline void csr_rows_r1(const DevMat &A, uint32_t b0, uint32_t b1, uint32_t e,
-                                   const double *__restrict__ x, const Acc &acc, uint32_t *s_st, uint32_t *s_bc,
-                                   int lane)
+// LDS of one wave besides its accumulator: a chunk's segments (COO blocks, or
+// the rows of CSR blocks that hold entries) and the mask of their ends.
+constexpr int kSegs = 4 * kWave;   // segments per chunk, four per lane
+constexpr int kMaskEnts = 2048;    // entries one mask covers
+// Any four COO blocks fit a mask: the cost model gives a block to COO only up
+// to 2s entries (2 lg(s) z + 2 lg(s) <= lg(s) z + (s + 1) 2 lg(s)).
+static_assert(4 * 2 * 256 <= kMaskEnts, "four COO blocks per mask");
+
+struct WaveLds {
+    uint32_t bc[kSegs];              // first column of every segment's block
+    uint64_t ends[kMaskEnts / 64];   // bit t: entry t is its segment's last
+    uint8_t to[kSegs];               // tiles: the block's strip within the tile; CSR: the row
+};
+
+// Values of segments' blocks [cb, cb + nbk) of a per-block array, four
+// consecutive blocks per lane (0 past the end): one 4- or 8- or 16-byte load
+// per lane, single ones in the last lane.
+template <typename T>
+__device__ __forceinline__ void load4(const T *__restrict__ a, uint32_t cb, uint32_t nbk, int lane, uint32_t (&v)[4])
 {
-    if (b0 >= b1) return;
-    const int s = A.s;
-    const int sw = s < kWave ? s : kWave;          // lanes per block
-    const int G = kWave / sw;                      // blocks per wave step
-    const int passes = s / sw;                     // row passes per block
-    const VT *__restrict__ val = static_cast<const VT *>(A.val[CSR]);
-    const uint8_t *__restrict__ ccol = A.csr_col;
-    const RT *__restrict__ rowptr = static_cast<const RT *>(A.csr_rowptr);
-#pragma unroll 1
-    for (uint32_t cb = b0; cb < b1; cb += kWave) {
-        const uint32_t jb = cb + lane;
-        const bool ok = jb < b1;
-        const uint32_t z = ok ? (uint32_t)A.z1[CSR][jb] + 1u : 0u;
-        const uint32_t incl = wave_incl_scan_dpp(z);
-        s_st[lane] = e + incl - z;
-        s_bc[lane] = ok ? (uint32_t)ld<BT>(A.bcol[CSR], jb) : 0u;
-        e += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-        wave_sync();
-        const int nbk = (int)min<uint32_t>(kWave, b1 - cb);
-        const int lb = lane / sw, lr = lane % sw;
-#pragma unroll 1
-        for (int j0 = 0; j0 < nbk; j0 += G) {
-            const int j = j0 + lb;
-            if (j < nbk) {
-                const RT *rp = rowptr + (uint64_t)(cb + (uint32_t)j) * (uint64_t)(s + 1);
-                const uint32_t st = s_st[j];
-                const int64_t xc = (int64_t)s_bc[j] * s;
-#pragma unroll 1
-                for (int ps = 0; ps < passes; ps++) {
-                    const int r = ps * sw + lr;
-                    const uint32_t q0 = rp[r], q1 = rp[r + 1];
-                    double hi = 0.0, lo = 0.0;
-                    uint32_t q = q0;
-                    for (; q + 1 < q1; q += 2) {
-                        const double v0 = (double)val[st + q], v1 = (double)val[st + q + 1];
-                        const double x0 = x[xc + ccol[st + q]], x1 = x[xc + ccol[st + q + 1]];
-                        acc_add<COMP>(hi, lo, v0, x0);
-                        acc_add<COMP>(hi, lo, v1, x1);
-                    }
-                    if (q < q1) acc_add<COMP>(hi, lo, (double)val[st + q], x[xc + ccol[st + q]]);
-                    if (q1 > q0) acc_atomic<COMP>(acc, (uint32_t)r, hi, lo);
-                }
+    const uint32_t j = 4u * (uint32_t)lane;
+    const T *__restrict__ p = a + cb + j;
+    T w[4] = {0, 0, 0, 0};
+    if (j + 4u <= nbk) {
+        __builtin_memcpy(w, p, sizeof(w));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (j + (uint32_t)i < nbk) w[i] = p[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = (uint32_t)w[i];
+}
+
+// How an entry's row and column follow from its index and its segment.
+enum SegMode { SEG_COO, SEG_TILE, SEG_CSR };
+
+// Windows of 64 consecutive entries from vp / ip on (values and in-block
+// indices: COO (lrow << k) | lcol, CSR lcol), T <= kMaskEnts entries in nseg
+// segments whose ends are marked in L.ends; `before` segments end before the
+// first one.  Values and indices are read 64 consecutive ones per load, U
+// windows in flight; an entry's segment is the number of end bits before it
+// (mbcnt over the window's mask word plus a running count).
+template <typename VT, typename IT, bool COMP, int MODE, int U>
+__device__ __forceinline__ void seg_windows(const VT *__restrict__ vp, const IT *__restrict__ ip, uint32_t T,
+                                            uint32_t nseg, uint32_t before, int k, const double *__restrict__ x,
+                                            const Acc &acc, const WaveLds &L, int lane_)
+{
+    const int lane = opaque_v(lane_);  // its addresses are not kept outside
+    const uint32_t smask = (1u << k) - 1u;
+    // W windows from entry q on; TAIL: the last of them is not full (its lanes
+    // past the last entry read that one again and add nothing)
+    auto windows = [&](uint32_t q, auto w_tag, auto tail_tag) __attribute__((always_inline)) {
+        constexpr int W = decltype(w_tag)::value;
+        constexpr bool TAIL = decltype(tail_tag)::value;
+        auto live = [&](int u) { return !(TAIL && u == W - 1) || q + (uint32_t)(u * kWave + lane) < T; };
+        uint32_t id[W], r[W];
+        double v[W], xv[W];
+#pragma unroll
+        for (int u = 0; u < W; u++) {
+            uint32_t t = (uint32_t)(u * kWave + lane);
+            if (TAIL && u == W - 1) t = min(t, T - 1u - q);
+            id[u] = (ip + q)[t];
+            v[u] = (double)(vp + q)[t];
+        }
+#pragma unroll
+        for (int u = 0; u < W; u++) {
+            const uint64_t m = L.ends[q / kWave + (uint32_t)u];
+            const uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
+            uint32_t own = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, before));
+            if (TAIL && u == W - 1) own = min(own, nseg - 1u);
+            before += (uint32_t)__popc(lo) + (uint32_t)__popc(hi);
+            if constexpr (MODE == SEG_CSR) {
+                r[u] = L.to[own];
+                xv[u] = x[L.bc[own] + id[u]];
+            } else {
+                r[u] = id[u] >> k;
+                if constexpr (MODE == SEG_TILE) r[u] += (uint32_t)L.to[own] << k;
+                xv[u] = x[L.bc[own] + (id[u] & smask)];
             }
         }
-        wave_sync();
+        if constexpr (COMP) {
+            // every returning add first, then the TwoSums and the compensation
+            // adds (hi and lo receive their adds in entry order either way):
+            // the returns are awaited once
+            double pr[W], pe[W], old[W];
+#pragma unroll
+            for (int u = 0; u < W; u++) {
+                pr[u] = prod<true>(v[u], xv[u], pe[u]);
+                if (live(u)) old[u] = atomicAdd(&acc.hi[r[u]], pr[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < W; u++)
+                if (live(u)) {
+                    double sum, err;
+                    two_sum(old[u], pr[u], sum, err);
+                    atomicAdd(&acc.lo[r[u]], err + pe[u]);
+                }
+        } else {
+#pragma unroll
+            for (int u = 0; u < W; u++)
+                if (live(u)) atomicAdd(&acc.hi[r[u]], v[u] * xv[u]);
+        }
+    };
+    using std::integral_constant;
+    uint32_t q = 0;
+#pragma unroll 1
+    for (; q + (uint32_t)(U * kWave) <= T; q += (uint32_t)(U * kWave))
+        windows(q, integral_constant<int, U>{}, std::false_type{});
+    const uint32_t left = T - q;  // uniform
+    if (U > 3 && left > 3u * kWave) windows(q, integral_constant<int, 4>{}, std::true_type{});
+    else if (U > 2 && left > 2u * kWave) windows(q, integral_constant<int, 3>{}, std::true_type{});
+    else if (U > 1 && left > (uint32_t)kWave) windows(q, integral_constant<int, 2>{}, std::true_type{});
+    else if (left) windows(q, integral_constant<int, 1>{}, std::true_type{});
+}
+
+// CSR group, blocks [b0, b1) whose first value is at offset e.  Chunks of 256
+// block rows (256 / s blocks), four consecutive rows of a block per lane: the
+// rows that hold entries are the chunk's segments (their number in L.to, the
+// block's first column in L.bc), the row pointers give their ends, and the
+// entries are taken as in the COO walk.
+// Bound: memory latency.  When the lane of a row walked the row's entries by
+// itself, one load of 3-entry rows touched 12 lines instead of 4 and waited
+// for the row pointers, and a long row held up the wave for its whole length
+// (R-MAT scale 20 s = 256 tiled, 10 % of the entries in CSR blocks, 128 -> 64
+// us; block_mix n = 2^22 s = 128 tiled 990 -> 686 us).
+template <typename VT, typename BT, typename RT, bool COMP>
+__device__ __forceinline__ void csr_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
+                                       const Acc &acc, WaveLds &L, int lane_)
+{
+    if (b0 >= b1) return;
+    const MatPtr A = opaque_s(A_);
+    const int lane = opaque_v(lane_);
+    const int k = A->k;
+    const VT *__restrict__ val = glob<VT>(A->val[CSR]);
+    const uint8_t *__restrict__ ccol = glob<uint8_t>(A->csr_col);
+    const RT *__restrict__ rowptr = glob<RT>(A->csr_rowptr);
+    const BT *__restrict__ bcol = glob<BT>(A->bcol[CSR]);
+    uint32_t *ends32 = reinterpret_cast<uint32_t *>(L.ends);
+    const uint32_t nb = (uint32_t)kSegs >> k;  // blocks per chunk (the cost model has no CSR blocks below s = 16)
+    const uint32_t j = (4u * (uint32_t)lane) >> k, r0 = (4u * (uint32_t)lane) & ((1u << k) - 1u);
+#pragma unroll 1
+    for (uint32_t cb = b0; cb < b1; cb += nb) {
+        uint32_t a[5] = {0, 0, 0, 0, 0}, bc = 0;
+        if (cb + j < b1) {
+            const RT *__restrict__ rp = rowptr + ((uint64_t)(cb + j) * (uint64_t)((1u << k) + 1u) + r0);
+            RT w[4];
+            __builtin_memcpy(w, rp, sizeof(w));
+#pragma unroll
+            for (int i = 0; i < 4; i++) a[i] = (uint32_t)w[i];
+            a[4] = (uint32_t)rp[4];
+            bc = (uint32_t)bcol[cb + j] << k;
+        }
+        // prefix sums of the entries (low half) and of the rows that hold some
+        uint32_t rows = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) rows += a[i + 1] != a[i];
+        const uint32_t mine = (a[4] - a[0]) | (rows << 16);
+        const uint32_t incl = wave_incl_scan_dpp(mine);
+        const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        const uint32_t T = tot & 0xFFFFu, nseg = tot >> 16;
+        // chunk positions of the rows' last entries, two per register (the
+        // cost model keeps a chunk's CSR blocks below 2^13 entries in all;
+        // none: 0xFFFF)
+        const uint32_t p0 = ((incl - mine) & 0xFFFFu) - a[0];
+        uint32_t o = (incl - mine) >> 16, last[2] = {~0u, ~0u};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (a[i + 1] != a[i]) {
+                L.bc[o] = bc;
+                L.to[o] = (uint8_t)(r0 + (uint32_t)i);
+                o++;
+                last[i / 2] ^= (0xFFFFu ^ (p0 + a[i + 1] - 1u)) << (16 * (i & 1));
+            }
+#pragma unroll 1
+        for (uint32_t w = 0; w < T; w += (uint32_t)kMaskEnts) {
+            const uint32_t Tw = min(T - w, (uint32_t)kMaskEnts);
+            ends32[lane] = 0u;
+            wave_sync();
+            uint32_t before = 0;  // rows that end before entry w
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t t = (last[i / 2] >> (16 * (i & 1))) & 0xFFFFu;
+                before += t < w;
+                if (t - w < Tw) atomicOr(&ends32[(t - w) >> 5], 1u << ((t - w) & 31u));
+            }
+            if (w) before = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan_dpp(before), kWave - 1);
+            wave_sync();
+            seg_windows<VT, uint8_t, COMP, SEG_CSR, 4>(val + (e + w), ccol + (e + w), Tw, nseg, before, k, x, acc, L,
+                                                       lane);
+            wave_sync();
+        }
+        e += T;
     }
 }
 
-// COO group, blocks [b0, b1) with first value at offset e.  Chunks of 64
-// blocks, lane j <-> block j.  Phase A: every lane handles the first ZS
-// entries of its own block (independent loads, no lookup); phase B, only when
-// some block of the chunk holds more than ZS entries: the remaining entries
-// are spread one per lane and located by a binary search over the chunk's
-// prefix sums in LDS.  A block's z1 holds z - 1 in its low A.zb bits and, in
-// a tile, the block's strip t within the tile above them: t << 2k is added to
-// its in-block indices, so (index >> k) = (t << k) + lrow is the tile row and
-// the column bits are unchanged.
-template <typename VT, typename BT, typename IT, bool COMP, int ZS, int CH, bool TILE = false>
-__device__ inline void coo_r1(const DevMat &A, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
-                              const Acc &acc, uint32_t *s_end, uint32_t *s_bc, uint32_t *s_st, uint32_t *s_to,
-                              int lane)
+// COO group, blocks [b0, b1) with first value at offset e.  Chunks of up to
+// 256 blocks (four per lane, one prefix sum) and 2048 entries; a block is a
+// segment: it sets the bit of its last entry in the LDS mask and leaves its
+// first column in LDS.  The chunk's entries are taken in storage order, at
+// addresses known before the block metadata arrive.  A block's z1 holds z - 1
+// in its low A.zb bits and, in a tile, the block's strip t within the tile
+// above them: the tile row is (t << k) + lrow.
+// Bound: memory latency and the x gathers.  Before, a binary search of the
+// prefix sums located every entry beyond a block's first two, which the
+// block's lane took by itself: 62 VALU instructions per 64 entries (28 now)
+// and loads that waited for the metadata.  With the CSR walk above: 27-point
+// stencil 160^3 s = 64 396 -> 262 us (4.4 TB/s), R-MAT scale 22 s = 256 tiled
+// 470 -> 354 us, scale 20 s = 64 210 -> 168 us.
+template <typename VT, typename BT, typename IT, bool COMP, bool TILE = false>
+__device__ __forceinline__ void coo_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
+                                       const Acc &acc, WaveLds &L, int lane_, bool sweep = false)
 {
     if (b0 >= b1) return;
-    const int s = A.s, k = A.k, zb = TILE ? A.zb : 16;
-    const uint32_t smask = (uint32_t)s - 1, zmask = (1u << zb) - 1u;
-    const VT *__restrict__ val = static_cast<const VT *>(A.val[COO]);
-    const IT *__restrict__ idx = static_cast<const IT *>(A.coo_idx);
-    const uint16_t *__restrict__ z1 = A.z1[COO];
-    const BT *__restrict__ bcol = static_cast<const BT *>(A.bcol[COO]);
-    // CH sub-chunks of 64 blocks per step: all their loads are issued before
-    // any of them is consumed, so several memory round trips overlap.
+    const MatPtr A = opaque_s(A_);
+    const int lane = opaque_v(lane_);
+    const int k = A->k, zb = TILE ? A->zb : 16;
+    const uint32_t zmask = (1u << zb) - 1u;
+    const VT *__restrict__ val = glob<VT>(A->val[COO]);
+    const IT *__restrict__ idx = glob<IT>(A->coo_idx);
+    const uint16_t *__restrict__ z1 = glob<uint16_t>(A->z1[COO]);
+    const BT *__restrict__ bcol = glob<BT>(A->bcol[COO]);
+    uint32_t *ends32 = reinterpret_cast<uint32_t *>(L.ends);
+    uint32_t cb = b0;
 #pragma unroll 1
-    for (uint32_t cb = b0; cb < b1; cb += (uint32_t)(kWave * CH)) {
-        // zt = z | (strip within the tile << 17)  (z <= 2^16)
-        uint32_t zt[CH], bc[CH], st[CH];
+    while (cb < b1) {
+        uint32_t nbk = min<uint32_t>(kSegs, b1 - cb);
+        uint32_t z[4], bc[4];
+        load4(z1, cb, nbk, lane, z);
+        load4(bcol, cb, nbk, lane, bc);
+        uint32_t to = 0, zs = 0;
 #pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const uint32_t jb = cb + (uint32_t)(c * kWave) + (uint32_t)lane;
-            const bool ok = jb < b1;
-            const uint32_t r = ok ? (uint32_t)z1[jb] : 0u;
-            if constexpr (TILE) zt[c] = ok ? ((r & zmask) + 1u) | ((r >> zb) << 17) : 0u;
-            else zt[c] = ok ? r + 1u : 0u;
-            bc[c] = ok ? (uint32_t)bcol[jb] : 0u;
-        }
-        auto zof = [&](int c) { return TILE ? zt[c] & 0x1FFFFu : zt[c]; };
-        auto tzof = [&](int c) { return TILE ? (zt[c] >> 17) << (2 * k) : 0u; };
-        const uint32_t e_step = e;
-#pragma unroll
-        for (int c = 0; c < CH; c++) {
-            const uint32_t incl = wave_incl_scan_dpp(zof(c));
-            st[c] = e + incl - zof(c);
-            e += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-        }
-        // blocks of 16 entries or more on average (a uniform decision): phase
-        // A would keep a few lanes busy for a whole memory round trip, so
-        // phase B takes every entry
-        const uint32_t nbs = min<uint32_t>(b1 - cb, (uint32_t)(kWave * CH));
-        const uint32_t za = (e - e_step >= 16u * nbs) ? 0u : (uint32_t)ZS;
-        if (za) {
-            uint32_t id[CH][ZS];
-            double v[CH][ZS], xv[CH][ZS];
-#pragma unroll
-            for (int c = 0; c < CH; c++)
-#pragma unroll
-                for (int i = 0; i < ZS; i++) {
-                    const bool h = (uint32_t)i < zof(c);
-                    id[c][i] = h ? (uint32_t)idx[st[c] + i] + tzof(c) : 0u;
-                    v[c][i] = h ? (double)val[st[c] + i] : 0.0;
-                }
-#pragma unroll
-            for (int c = 0; c < CH; c++)
-#pragma unroll
-                for (int i = 0; i < ZS; i++)
-                    xv[c][i] = ((uint32_t)i < zof(c)) ? x[(int64_t)bc[c] * s + (id[c][i] & smask)] : 0.0;
-#pragma unroll
-            for (int c = 0; c < CH; c++)
-#pragma unroll
-                for (int i = 0; i < ZS; i++)
-                    if ((uint32_t)i < zof(c)) {
-                        double pe;
-                        const double p = prod<COMP>(v[c][i], xv[c][i], pe);
-                        acc_atomic<COMP>(acc, id[c][i] >> k, p, pe);
-                    }
-        }
-        // phase B: entries beyond the first za of a block, one per lane
-#pragma unroll 1
-        for (int c = 0; c < CH; c++) {
-            const uint32_t rem = zof(c) > za ? zof(c) - za : 0u;
-            if (__ballot(rem != 0) == 0) continue;
-            const uint32_t rincl = wave_incl_scan_dpp(rem);
-            const uint32_t RT = (uint32_t)__builtin_amdgcn_readlane((int)rincl, kWave - 1);
-            s_end[lane] = rincl;
-            s_bc[lane] = bc[c];
-            s_st[lane] = st[c] + za;
-            if constexpr (TILE) s_to[lane] = tzof(c);
-            wave_sync();
-            const uint32_t cs = cb + (uint32_t)(c * kWave);
-            const int nbk = (int)min<uint32_t>(kWave, b1 - cs);
-            // two windows of 64 entries per step: both searches, then all
-            // loads, then the updates
-#pragma unroll 1
-            for (uint32_t q = 0; q < RT; q += 2 * kWave) {
-                uint32_t pos[2], xb[2], ide[2], rb[2];
-                double ve[2], xe[2];
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const uint32_t t = q + (uint32_t)(u * kWave + lane);
-                    int lo = 0, hi = nbk - 1;
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if (s_end[mid] > t) hi = mid; else lo = mid + 1;
-                    }
-                    pos[u] = s_st[lo] + t - (lo ? s_end[lo - 1] : 0u);
-                    xb[u] = s_bc[lo];
-                    rb[u] = TILE ? s_to[lo] : 0u;
-                }
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const bool h = q + (uint32_t)(u * kWave + lane) < RT;
-                    ide[u] = h ? (uint32_t)idx[pos[u]] + rb[u] : 0u;
-                    ve[u] = h ? (double)val[pos[u]] : 0.0;
-                }
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const bool h = q + (uint32_t)(u * kWave + lane) < RT;
-                    xe[u] = h ? x[(int64_t)xb[u] * s + (ide[u] & smask)] : 0.0;
-                }
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-                    if (q + (uint32_t)(u * kWave + lane) < RT) {
-                        double pe;
-                        const double p = prod<COMP>(ve[u], xe[u], pe);
-                        acc_atomic<COMP>(acc, ide[u] >> k, p, pe);
-                    }
+        for (int i = 0; i < 4; i++) {
+            if constexpr (TILE) {
+                to |= (z[i] >> zb) << (8 * i);
+                z[i] &= zmask;
             }
-            wave_sync();
+            z[i] = 4u * (uint32_t)lane + (uint32_t)i < nbk ? z[i] + 1u : 0u;
+            zs += z[i];
+            bc[i] <<= k;
         }
+        const uint32_t incl = wave_incl_scan_dpp(zs);
+        uint32_t T = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        bool mine = true;
+        if (T > (uint32_t)kMaskEnts) {  // uniform: take the lanes whose blocks fit
+            mine = incl <= (uint32_t)kMaskEnts;
+            const int nl = __popcll(__ballot(mine));
+            T = (uint32_t)__builtin_amdgcn_readlane((int)incl, nl - 1);
+            nbk = min(nbk, 4u * (uint32_t)nl);
+        }
+        *reinterpret_cast<uint4 *>(&L.bc[4 * lane]) = make_uint4(bc[0], bc[1], bc[2], bc[3]);
+        if constexpr (TILE) *reinterpret_cast<uint32_t *>(&L.to[4 * lane]) = to;
+        ends32[lane] = 0u;
+        wave_sync();
+        uint32_t p = incl - zs;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            p += z[i];
+            if (z[i] && mine) atomicOr(&ends32[(p - 1u) >> 5], 1u << ((p - 1u) & 31u));
+        }
+        wave_sync();
+        // one window in flight keeps the tiles' common sweep of a large x
+        // together (Balance::tile_sweep)
+        if (TILE && sweep)
+            seg_windows<VT, IT, COMP, SEG_TILE, 1>(val + e, idx + e, T, nbk, 0u, k, x, acc, L, lane);
+        else
+            seg_windows<VT, IT, COMP, TILE ? SEG_TILE : SEG_COO, 4>(val + e, idx + e, T, nbk, 0u, k, x, acc, L, lane);
+        wave_sync();
+        e += T;
+        cb += nbk;
     }
 }
 
@@ -317,21 +438,23 @@ __device__ inline void coo_r1(const DevMat &A, uint32_t b0, uint32_t b1, uint32_
 // products in registers, the P lanes of a row are summed with DPP, and the
 // first lane of the row adds the sum to the strip accumulator.
 template <typename VT, typename BT, bool COMP>
-__device__ inline void bmdn_r1(const DevMat &A, int sc, uint32_t b0, uint32_t b1, uint64_t vb,
-                               const double *__restrict__ x, const Acc &acc, int lane)
+__device__ __forceinline__ void bmdn_r1(MatPtr A_, int sc, uint32_t b0, uint32_t b1, uint64_t vb,
+                               const double *__restrict__ x, const Acc &acc, int lane_)
 {
     if (b0 >= b1) return;
-    const int s = A.s, k = A.k;
+    const MatPtr A = opaque_s(A_);
+    const int lane = opaque_v(lane_);
+    const int s = A->s, k = A->k;
     const uint32_t ss = (uint32_t)s * (uint32_t)s;
     const uint32_t cw = s >= 64 ? (uint32_t)s : (ss >= 64 ? ss / 64 : 1u);
     const int npass = (int)((ss + 64u * cw - 1) / (64u * cw));
     const int P = (int)((uint32_t)s / cw);
-    const int64_t n = A.n;
-    const VT *__restrict__ val = static_cast<const VT *>(A.val[sc]);
+    const int64_t n = A->n;
+    const VT *__restrict__ val = glob<VT>(A->val[sc]);
 #pragma unroll 1
     for (uint32_t b = b0; b < b1; b++) {
-        const int64_t c0 = (int64_t)ld<BT>(A.bcol[sc], b) * s;
-        const uint64_t *__restrict__ words = A.bm_words + (uint64_t)b * A.W;
+        const int64_t c0 = (int64_t)glob<BT>(A->bcol[sc])[b] * s;
+        const uint64_t *__restrict__ words = glob<uint64_t>(A->bm_words) + (uint64_t)b * A->W;
         const uint64_t db = (uint64_t)b * ss;
 #pragma unroll 1
         for (int q = 0; q < npass; q++) {
@@ -433,14 +556,16 @@ __device__ inline void bmdn_r1(const DevMat &A, int sc, uint32_t b0, uint32_t b1
 // summed with DPP at the end.  (Lanes owning S*S/64 consecutive positions
 // made a load touch up to 64 lines: S = 32 streamed 3.8 TB/s, now 5.6.)
 template <typename BT, int S>
-__device__ inline void dense_coal_r1(const DevMat &A, uint32_t b0, uint32_t b1, const double *__restrict__ x,
-                                     const Acc &acc, int lane)
+__device__ __forceinline__ void dense_coal_r1(MatPtr A_, uint32_t b0, uint32_t b1, const double *__restrict__ x,
+                                     const Acc &acc, int lane_)
 {
     static_assert(S == 16 || S == 32, "S x S blocks of whole 128-position steps");
     constexpr int L = S / 2, NQ = S * S / 128, RQ = 128 / S;
     if (b0 >= b1) return;
-    const double *__restrict__ val = static_cast<const double *>(A.val[DENSE]);
-    const int64_t n = A.n;
+    const MatPtr A = opaque_s(A_);
+    const int lane = opaque_v(lane_);
+    const double *__restrict__ val = glob<double>(A->val[DENSE]);
+    const int64_t n = A->n;
     const int cl = 2 * (lane % L);
     const bool xal = x_aligned16(x);  // wave-uniform: x pairs as double2 loads or two scalar loads
     double a[NQ];
@@ -448,7 +573,7 @@ __device__ inline void dense_coal_r1(const DevMat &A, uint32_t b0, uint32_t b1, 
     for (int q = 0; q < NQ; q++) a[q] = 0.0;
 #pragma unroll 1
     for (uint32_t b = b0; b < b1; b++) {
-        const int64_t c0 = (int64_t)ld<BT>(A.bcol[DENSE], b) * S + cl;
+        const int64_t c0 = (int64_t)glob<BT>(A->bcol[DENSE])[b] * S + cl;
         double x0 = 0.0, x1 = 0.0;  // columns past n hold stored zeros; x is not read there
         if (c0 + 1 < n && !xal) {
             x0 = x[c0];
@@ -484,17 +609,17 @@ __device__ inline void dense_coal_r1(const DevMat &A, uint32_t b0, uint32_t b1, 
 // at compile time (u8 indices with u16 row pointers: s = 16; u16 indices:
 // s >= 32), so each kernel carries only the path it can take.
 template <typename VT, typename BT, typename IT, typename RT, bool COMP>
-__device__ inline void dense_r1(const DevMat &A, uint32_t b0, uint32_t b1, const double *__restrict__ x,
+__device__ __forceinline__ void dense_r1(MatPtr A, uint32_t b0, uint32_t b1, const double *__restrict__ x,
                                 const Acc &acc, int lane)
 {
     if constexpr (sizeof(VT) == 8 && !COMP && sizeof(IT) == 2) {
-        if (A.s == 32) {
+        if (A->s == 32) {
             dense_coal_r1<BT, 32>(A, b0, b1, x, acc, lane);
             return;
         }
     }
     if constexpr (sizeof(VT) == 8 && !COMP && sizeof(IT) == 1 && sizeof(RT) == 2) {
-        if (A.s == 16) {
+        if (A->s == 16) {
             dense_coal_r1<BT, 16>(A, b0, b1, x, acc, lane);
             return;
         }
@@ -527,94 +652,77 @@ __device__ inline int64_t xcd_block_id()
 // TL: 0 the matrix is not tiled, 1 it is, 2 either (read from B.tiled); the
 // single-matrix kernels are compiled for 0 or 1 so that each carries only one
 // of the light-item paths (scalar-register pressure).
-template <typename VT, typename BT, typename IT, typename RT, bool COMP, int ZS = 2, int CH = 4, int TL = 2>
-__device__ inline void spmv_item(const DevMat &A, const Balance &B, int64_t item, const double *__restrict__ x,
-                                 double *__restrict__ y, double alpha, double beta, double *acc_buf,
-                                 uint32_t *s_end, uint32_t *s_bc, uint32_t *s_st, uint32_t *s_to, int lane)
+template <typename VT, typename BT, typename IT, typename RT, bool COMP, int TL = 2>
+__device__ __forceinline__ void spmv_item(MatPtr A, BalPtr B, int64_t item, const double *__restrict__ x,
+                                 double *__restrict__ y, double alpha, double beta, double *acc_buf, WaveLds &L,
+                                 int lane)
 {
-    const int s = A.s;
+    const int s = A->s;
     Acc acc;
     acc.hi = acc_buf;
     acc.lo = COMP ? acc_buf + 256 : nullptr;
-    for (int i = lane; i < s; i += kWave) {
-        acc.hi[i] = 0.0;
-        if constexpr (COMP) acc.lo[i] = 0.0;
-    }
-    wave_sync();
-    if (item < B.n_light) {
+    auto clear = [&](int rows) {
+        for (int i = lane; i < rows; i += kWave) {
+            acc.hi[i] = 0.0;
+            if constexpr (COMP) acc.lo[i] = 0.0;
+        }
+        wave_sync();
+    };
+    if (item < B->n_light) {
         // light item: light strips at positions [p0, p1) of the light list
         uint32_t p0 = (uint32_t)item, p1 = (uint32_t)item + 1u;
-        if (B.pack) {
-            p0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)B.pack[item]);
-            p1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)B.pack[item + 1]);
+        if (B->pack) {
+            p0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)glob<uint32_t>(B->pack)[item]);
+            p1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)glob<uint32_t>(B->pack)[item + 1]);
         }
-        const bool tiled = TL == 1 || (TL == 2 && B.tiled);
+        const bool tiled = TL == 1 || (TL == 2 && B->tiled);
+        uint32_t tb0 = 0, tb1 = 0, te0 = 0;  // tiled: the item's COO blocks
         if (tiled) {
-            // the item's strips light[p0 .. p1): one pass over their COO
-            // blocks (rows (position << k) + lrow), then each strip's CSR /
-            // bitmap / dense groups, then all rows
-            const uint32_t *R = B.coo_rng + (uint64_t)item * 3;
-            const uint32_t cb0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[0]);
-            const uint32_t cb1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[1]);
-            const uint32_t ce0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[2]);
+            const uint32_t *R = glob<uint32_t>(B->coo_rng) + (uint64_t)item * 3;
+            tb0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[0]);
+            tb1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[1]);
+            te0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[2]);
             const int T = (int)(p1 - p0);
-            const int rows = T * s;
-            for (int i = s + lane; i < rows; i += kWave) {
-                acc.hi[i] = 0.0;
-                if constexpr (COMP) acc.lo[i] = 0.0;
-            }
-            wave_sync();
-            if (T > 1)
-                coo_r1<VT, BT, IT, COMP, ZS, CH, true>(A, cb0, cb1, ce0, x, acc, s_end, s_bc, s_st, s_to, lane);
-            else
-                coo_r1<VT, BT, IT, COMP, ZS, CH>(A, cb0, cb1, ce0, x, acc, s_end, s_bc, s_st, s_to, lane);
-#pragma unroll 1
-            for (int t = 0; t < T; t++) {
-                const int64_t I = (int64_t)__builtin_amdgcn_readfirstlane((int)B.light[p0 + (uint32_t)t]);
-                Acc at;
-                at.hi = acc.hi + t * s;
-                at.lo = COMP ? acc.lo + t * s : nullptr;
-                csr_rows_r1<VT, BT, RT, COMP>(A, A.sptr[CSR][I], A.sptr[CSR][I + 1], A.eptr[CSR][I], x, at, s_st,
-                                              s_bc, lane);
-                wave_sync();
-                bmdn_r1<VT, BT, COMP>(A, BITMAP, A.sptr[BITMAP][I], A.sptr[BITMAP][I + 1], A.eptr[BITMAP][I], x,
-                                      at, lane);
-                dense_r1<VT, BT, IT, RT, COMP>(A, A.sptr[DENSE][I], A.sptr[DENSE][I + 1], x, at, lane);
-                wave_sync();
-            }
-            for (int r = lane; r < rows; r += kWave) {
-                const int64_t gr = (int64_t)B.light[p0 + (uint32_t)(r >> A.k)] * s + (r & (s - 1));
-                if (gr < A.m) {
-                    double a = acc.hi[r];
-                    if constexpr (COMP) a += acc.lo[r];
-                    y[gr] = (beta == 0.0) ? alpha * a : alpha * a + beta * y[gr];
+            if (T > 1) {
+                // a tile of strips that hold COO blocks only: one pass over
+                // them (rows (position << k) + lrow), then all rows
+                const int rows = T * s;
+                clear(rows);
+                coo_r1<VT, BT, IT, COMP, true>(A, tb0, tb1, te0, x, acc, L, lane, B->tile_sweep);
+                for (int r = lane; r < rows; r += kWave) {
+                    const int64_t gr = (int64_t)glob<uint32_t>(B->light)[p0 + (uint32_t)(r >> A->k)] * s + (r & (s - 1));
+                    if (gr < A->m) {
+                        double a = acc.hi[r];
+                        if constexpr (COMP) a += acc.lo[r];
+                        y[gr] = (beta == 0.0) ? alpha * a : alpha * a + beta * y[gr];
+                    }
                 }
+                wave_sync();
+                return;
             }
-            wave_sync();
-            return;
         }
 #pragma unroll 1
         for (uint32_t p = p0; p < p1; p++) {
-            const int64_t I = B.light ? (int64_t)__builtin_amdgcn_readfirstlane((int)B.light[p]) : (int64_t)p;
-            if (p != p0) {  // the previous strip's rows are written; clear for this one
-                for (int i = lane; i < s; i += kWave) {
-                    acc.hi[i] = 0.0;
-                    if constexpr (COMP) acc.lo[i] = 0.0;
-                }
-                wave_sync();
+            const int64_t I = B->light ? (int64_t)__builtin_amdgcn_readfirstlane((int)glob<uint32_t>(B->light)[p]) : (int64_t)p;
+            // all group bounds first: one round trip
+            if (!tiled) {
+                tb0 = glob<uint32_t>(A->sptr[COO])[I];
+                tb1 = glob<uint32_t>(A->sptr[COO])[I + 1];
+                te0 = glob<uint32_t>(A->eptr[COO])[I];
             }
-            coo_r1<VT, BT, IT, COMP, ZS, CH>(A, A.sptr[COO][I], A.sptr[COO][I + 1], A.eptr[COO][I], x, acc, s_end, s_bc,
-                                             s_st, s_to, lane);
-            csr_rows_r1<VT, BT, RT, COMP>(A, A.sptr[CSR][I], A.sptr[CSR][I + 1], A.eptr[CSR][I], x, acc, s_st, s_bc,
-                                          lane);
+            const uint32_t r0 = glob<uint32_t>(A->sptr[CSR])[I], r1 = glob<uint32_t>(A->sptr[CSR])[I + 1], re = glob<uint32_t>(A->eptr[CSR])[I];
+            const uint32_t m0 = glob<uint32_t>(A->sptr[BITMAP])[I], m1 = glob<uint32_t>(A->sptr[BITMAP])[I + 1], me = glob<uint32_t>(A->eptr[BITMAP])[I];
+            const uint32_t d0 = glob<uint32_t>(A->sptr[DENSE])[I], d1 = glob<uint32_t>(A->sptr[DENSE])[I + 1];
+            clear(s);
+            coo_r1<VT, BT, IT, COMP>(A, tb0, tb1, te0, x, acc, L, lane);
+            csr_r1<VT, BT, RT, COMP>(A, r0, r1, re, x, acc, L, lane);
             wave_sync();
-            bmdn_r1<VT, BT, COMP>(A, BITMAP, A.sptr[BITMAP][I], A.sptr[BITMAP][I + 1], A.eptr[BITMAP][I], x, acc,
-                                  lane);
-            dense_r1<VT, BT, IT, RT, COMP>(A, A.sptr[DENSE][I], A.sptr[DENSE][I + 1], x, acc, lane);
+            bmdn_r1<VT, BT, COMP>(A, BITMAP, m0, m1, me, x, acc, lane);
+            dense_r1<VT, BT, IT, RT, COMP>(A, d0, d1, x, acc, lane);
             wave_sync();
             for (int r = lane; r < s; r += kWave) {
                 const int64_t gr = I * s + r;
-                if (gr >= A.m) break;
+                if (gr >= A->m) break;
                 double a = acc.hi[r];
                 if constexpr (COMP) a += acc.lo[r];
                 y[gr] = (beta == 0.0) ? alpha * a : alpha * a + beta * y[gr];
@@ -622,25 +730,23 @@ __device__ inline void spmv_item(const DevMat &A, const Balance &B, int64_t item
             wave_sync();
         }
     } else {
-        const int64_t u = item - B.n_light;
-        const uint32_t *U = B.units + u * 4;
+        const int64_t u = item - B->n_light;
+        const uint32_t *U = glob<uint32_t>(B->units) + u * 4;
         const uint32_t sc = U[0] & 3u, b0 = U[1], b1 = U[2], e0 = U[3];
+        clear(s);
         // constant scheme arguments: the descriptor's per-scheme arrays are
         // then indexed statically (a runtime index would force a local copy
         // of the descriptor, as in the batched kernel, into scratch memory)
-        // the tiled kernel's units take one entry per block in phase A (its
-        // tiles keep ZS): R-MAT scale 22 s = 64 / 128 / 256 0.623 / 0.590 /
-        // 0.536 -> 0.611 / 0.584 / 0.528 ms, same registers
         if (sc == COO)
-            coo_r1<VT, BT, IT, COMP, (TL == 1 ? 1 : ZS), CH>(A, b0, b1, e0, x, acc, s_end, s_bc, s_st, s_to, lane);
+            coo_r1<VT, BT, IT, COMP>(A, b0, b1, e0, x, acc, L, lane);
         else if (sc == CSR)
-            csr_rows_r1<VT, BT, RT, COMP>(A, b0, b1, e0, x, acc, s_st, s_bc, lane);
+            csr_r1<VT, BT, RT, COMP>(A, b0, b1, e0, x, acc, L, lane);
         else if (sc == BITMAP)
             bmdn_r1<VT, BT, COMP>(A, BITMAP, b0, b1, e0, x, acc, lane);
         else
             dense_r1<VT, BT, IT, RT, COMP>(A, b0, b1, x, acc, lane);
         wave_sync();
-        double *part = B.part + u * (size_t)s * (COMP ? 2 : 1);
+        double *part = glob_rw(B->part) + u * (size_t)s * (COMP ? 2 : 1);
         for (int r = lane; r < s; r += kWave) {
             part[r] = acc.hi[r];
             if constexpr (COMP) part[s + r] = acc.lo[r];
@@ -654,29 +760,35 @@ __device__ inline void spmv_item(const DevMat &A, const Balance &B, int64_t item
 // light) -- whose rows are written to y; items n_light + u are
 // units u of heavy strips: one scheme group's block range, whose partial sums
 // go to part[u] and are combined by k_spmv_fixup.
-template <typename VT, typename BT, typename IT, typename RT, bool COMP, int ZS, int CH, bool TILED>
-__global__ __launch_bounds__(64 * kStripWaves) void k_spmv_strip(DevMat A, const double *__restrict__ x,
-                                                                 double *__restrict__ y, double alpha, double beta,
-                                                                 Balance B)
+struct StripArgs {
+    DevMat A;
+    Balance B;
+    const double *x;
+    double *y;
+    double alpha, beta;
+};
+
+template <typename VT, typename BT, typename IT, typename RT, bool COMP, bool TILED>
+__global__ __launch_bounds__(64 * kStripWaves) void k_spmv_strip(StripArgs)
 {
     constexpr int kWaves = kStripWaves;
     // s rows, or a tile's (kTileRows; kTileRowsComp compensated, lo half at +256)
-    static_assert(kTileRowsComp == 256 && kTileRows >= 256, "accumulator layout");
-    __shared__ double s_acc[kWaves][COMP ? 512 : kTileRows];
-    __shared__ uint32_t s_end[kWaves][kWave];
-    __shared__ uint32_t s_bc[kWaves][kWave];
-    __shared__ uint32_t s_st[kWaves][kWave];
-    __shared__ uint32_t s_to[kWaves][kWave];
+    static_assert(kTileRowsComp == 256 && kTileRows >= 512, "accumulator layout");
+    __shared__ double s_acc[kWaves][kTileRows];
+    __shared__ __align__(16) WaveLds s_lds[kWaves];
+    // the arguments, where the launch put them (the struct is the only one)
+    const auto *P = (const __attribute__((address_space(4))) StripArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    const BalPtr B = &P->B;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     int64_t item = xcd_block_id() * kWaves + wave;
-    if (B.order) {  // a slot table (column panels: items per XCD; tiles: launch order)
-        const uint32_t o = B.order[(int64_t)blockIdx.x * kWaves + wave];
+    if (B->order) {  // a slot table (column panels: items per XCD; tiles: launch order)
+        const uint32_t o = glob<uint32_t>(B->order)[(int64_t)blockIdx.x * kWaves + wave];
         if (o == kNoItem) return;
         item = (int64_t)__builtin_amdgcn_readfirstlane((int)o);
     }
-    if (item >= B.n_light + B.n_units) return;  // whole wave leaves; no workgroup barriers below
-    spmv_item<VT, BT, IT, RT, COMP, ZS, CH, TILED ? 1 : 0>(A, B, item, x, y, alpha, beta, s_acc[wave], s_end[wave],
-                                                           s_bc[wave], s_st[wave], s_to[wave], lane);
+    if (item >= B->n_light + B->n_units) return;  // whole wave leaves; no workgroup barriers below
+    spmv_item<VT, BT, IT, RT, COMP, TILED ? 1 : 0>(&P->A, B, item, glob<double>(P->x), glob_rw(P->y), P->alpha,
+                                                   P->beta, s_acc[wave], s_lds[wave], lane);
 }
 
 // ===========================================================================
@@ -805,59 +917,6 @@ __global__ __launch_bounds__(256) void k_spmv_trans(DevMat A, Balance B, const d
     }
 }
 
-// A wave-uniform table field, read through the constant address space (the
-// table does not change during a launch): a scalar load into SGPRs.
-template <typename T>
-__device__ inline T ld_const(const T *p)
-{
-    return *(const __attribute__((address_space(4))) T *)p;
-}
-
-// Copy of a batch table entry, field by field (a word-wise copy through a
-// cast pointer kept the whole entry in per-lane scratch memory).
-__device__ inline BatchEntry load_entry(const BatchEntry *p)
-{
-    BatchEntry e;
-    e.A.m = ld_const(&p->A.m);
-    e.A.n = ld_const(&p->A.n);
-    e.A.M = ld_const(&p->A.M);
-    e.A.N = ld_const(&p->A.N);
-    e.A.s = ld_const(&p->A.s);
-    e.A.k = ld_const(&p->A.k);
-    e.A.W = ld_const(&p->A.W);
-    e.A.zb = ld_const(&p->A.zb);
-#pragma unroll
-    for (int x = 0; x < 4; x++) {
-        e.A.sptr[x] = ld_const(&p->A.sptr[x]);
-        e.A.eptr[x] = ld_const(&p->A.eptr[x]);
-        e.A.bcol[x] = ld_const(&p->A.bcol[x]);
-        e.A.z1[x] = ld_const(&p->A.z1[x]);
-        e.A.val[x] = ld_const(&p->A.val[x]);
-    }
-    e.A.coo_idx = ld_const(&p->A.coo_idx);
-    e.A.csr_rowptr = ld_const(&p->A.csr_rowptr);
-    e.A.csr_col = ld_const(&p->A.csr_col);
-    e.A.bm_words = ld_const(&p->A.bm_words);
-    e.B.light = ld_const(&p->B.light);
-    e.B.pack = ld_const(&p->B.pack);
-    e.B.units = ld_const(&p->B.units);
-    e.B.heavy = ld_const(&p->B.heavy);
-    e.B.part = ld_const(&p->B.part);
-    e.B.order = ld_const(&p->B.order);
-    e.B.n_light = ld_const(&p->B.n_light);
-    e.B.n_units = ld_const(&p->B.n_units);
-    e.B.n_heavy = ld_const(&p->B.n_heavy);
-    e.B.n_slots = ld_const(&p->B.n_slots);
-    e.B.tiled = ld_const(&p->B.tiled);
-    e.B.coo_rng = ld_const(&p->B.coo_rng);
-    e.x = ld_const(&p->x);
-    e.y = ld_const(&p->y);
-    e.item0 = ld_const(&p->item0);
-    e.code = ld_const(&p->code);
-    e.comp = ld_const(&p->comp);
-    return e;
-}
-
 // Many matrices in one launch: the waves take the global items [0, G), wave w
 // items w, w + W, ... (W = all waves of the grid); item_mat[g] names the
 // matrix of item g, whose index-type combination (batch_code) selects the
@@ -874,50 +933,40 @@ __global__ __launch_bounds__(256, 6) void k_batch_spmv(const BatchEntry *__restr
 {
     using VT = typename std::conditional<COMP, float, double>::type;
     constexpr int kWaves = 4;
-    static_assert(kTileRows >= 2 * kTileRowsComp, "compensated accumulators: hi and lo halves");
     __shared__ double s_acc[kWaves][kTileRows];
-    __shared__ uint32_t s_end[kWaves][kWave];
-    __shared__ uint32_t s_bc[kWaves][kWave];
-    __shared__ uint32_t s_st[kWaves][kWave];
-    __shared__ uint32_t s_to[kWaves][kWave];
+    __shared__ __align__(16) WaveLds s_lds[kWaves];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t nw = (int64_t)gridDim.x * kWaves;
 #pragma unroll 1
     for (int64_t g = g0 + (int64_t)blockIdx.x * kWaves + wave; g < G; g += nw) {
         const int mat = __builtin_amdgcn_readfirstlane((int)item_mat[g]);
-        // the table is read-only during the launch: its fields are read through
-        // the constant address space (scalar loads into SGPRs, as the
-        // single-matrix kernel gets them from its arguments)
-        const BatchEntry e = load_entry(E + mat);
+        // the table is read-only during the launch: constant address space
+        const auto *e = (const __attribute__((address_space(4))) BatchEntry *)(E + mat);
+        const double *x = glob<double>(e->x);
+        double *y = glob_rw(e->y);
         long long t0 = 0;
         if constexpr (TIMED) t0 = clock64();
-        const int64_t it = g - e.item0;
+        const int64_t it = g - e->item0;
         double *sa = s_acc[wave];
-        uint32_t *se = s_end[wave], *sb = s_bc[wave], *ss = s_st[wave], *so = s_to[wave];
-        switch (e.code) {  // batch_code: (bcol u32 ? 3 : 0) + (s <= 8 ? 0 : s <= 16 ? 1 : 2)
+        WaveLds &sl = s_lds[wave];
+        switch (e->code) {  // batch_code: (bcol u32 ? 3 : 0) + (s <= 8 ? 0 : s <= 16 ? 1 : 2)
         case 0:
-            spmv_item<VT, uint16_t, uint8_t, uint8_t, COMP>(e.A, e.B, it, e.x, e.y, alpha, beta, sa, se, sb,
-                                                                 ss, so, lane);
+            spmv_item<VT, uint16_t, uint8_t, uint8_t, COMP>(&e->A, &e->B, it, x, y, alpha, beta, sa, sl, lane);
             break;
         case 1:
-            spmv_item<VT, uint16_t, uint8_t, uint16_t, COMP>(e.A, e.B, it, e.x, e.y, alpha, beta, sa, se, sb,
-                                                                  ss, so, lane);
+            spmv_item<VT, uint16_t, uint8_t, uint16_t, COMP>(&e->A, &e->B, it, x, y, alpha, beta, sa, sl, lane);
             break;
         case 2:
-            spmv_item<VT, uint16_t, uint16_t, uint16_t, COMP>(e.A, e.B, it, e.x, e.y, alpha, beta, sa, se,
-                                                                   sb, ss, so, lane);
+            spmv_item<VT, uint16_t, uint16_t, uint16_t, COMP>(&e->A, &e->B, it, x, y, alpha, beta, sa, sl, lane);
             break;
         case 3:
-            spmv_item<VT, uint32_t, uint8_t, uint8_t, COMP>(e.A, e.B, it, e.x, e.y, alpha, beta, sa, se, sb,
-                                                                 ss, so, lane);
+            spmv_item<VT, uint32_t, uint8_t, uint8_t, COMP>(&e->A, &e->B, it, x, y, alpha, beta, sa, sl, lane);
             break;
         case 4:
-            spmv_item<VT, uint32_t, uint8_t, uint16_t, COMP>(e.A, e.B, it, e.x, e.y, alpha, beta, sa, se, sb,
-                                                                  ss, so, lane);
+            spmv_item<VT, uint32_t, uint8_t, uint16_t, COMP>(&e->A, &e->B, it, x, y, alpha, beta, sa, sl, lane);
             break;
         default:
-            spmv_item<VT, uint32_t, uint16_t, uint16_t, COMP>(e.A, e.B, it, e.x, e.y, alpha, beta, sa, se,
-                                                                   sb, ss, so, lane);
+            spmv_item<VT, uint32_t, uint16_t, uint16_t, COMP>(&e->A, &e->B, it, x, y, alpha, beta, sa, sl, lane);
             break;
         }
         if constexpr (TIMED) {
@@ -1562,36 +1611,8 @@ void launch_t(const DevMat &A, const double *X, int64_t ldx, double *Y, int64_t 
     ABHSF_HIP(hipGetLastError());
 }
 
-template <typename VT, typename BT, typename IT, typename RT, bool COMP, bool TILED>
-void launch_strip(const DevMat &A, const Balance &b, int64_t nblk, bool coo_single, const double *x, double *y,
-                  double alpha, double beta, hipStream_t st)
-{
-    // COO blocks of (almost) one entry: phase A takes one entry from each of
-    // 8 x 64 blocks per step (more gathers in flight, no unused entry slot);
-    // otherwise two entries from each of 4 x 64 blocks.  Tiles always take
-    // the 4 x 64 steps: a tile's COO stream advances through x in smaller
-    // column ranges per step (block_mix 0.480 -> 0.474 ms, uniform scatter
-    // 0.624 -> 0.606 ms).
-    if constexpr (!TILED) {
-        if (coo_single) {
-            hipLaunchKernelGGL((k_spmv_strip<VT, BT, IT, RT, COMP, 1, 8, false>), dim3((unsigned)nblk),
-                               dim3(64 * kStripWaves), 0, st, A, x, y, alpha, beta, b);
-            return;
-        }
-    }
-    if constexpr (TILED) {
-        if (b.tile_zs1) {
-            hipLaunchKernelGGL((k_spmv_strip<VT, BT, IT, RT, COMP, 1, 4, true>), dim3((unsigned)nblk),
-                               dim3(64 * kStripWaves), 0, st, A, x, y, alpha, beta, b);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((k_spmv_strip<VT, BT, IT, RT, COMP, 2, 4, TILED>), dim3((unsigned)nblk), dim3(64 * kStripWaves),
-                       0, st, A, x, y, alpha, beta, b);
-}
-
 template <typename VT, typename BT, typename IT, typename RT, bool COMP>
-void launch_spmv(const DevMat &A, const Balance &B, bool coo_single, const double *x, double *y, double alpha,
+void launch_spmv(const DevMat &A, const Balance &B, const double *x, double *y, double alpha,
                  double beta, hipStream_t st)
 {
     if (A.M == 0) return;
@@ -1603,10 +1624,13 @@ void launch_spmv(const DevMat &A, const Balance &B, bool coo_single, const doubl
     // tiled matrices have their own kernels (each carries one light-item
     // path); the choice is made once, here: a tiled storage read by an untiled
     // kernel would take its z1 strip bits for entry counts
+    const StripArgs args{A, b, x, y, alpha, beta};
     if (b.tiled)
-        launch_strip<VT, BT, IT, RT, COMP, true>(A, b, nblk, coo_single, x, y, alpha, beta, st);
+        hipLaunchKernelGGL((k_spmv_strip<VT, BT, IT, RT, COMP, true>), dim3((unsigned)nblk), dim3(64 * kStripWaves), 0,
+                           st, args);
     else
-        launch_strip<VT, BT, IT, RT, COMP, false>(A, b, nblk, coo_single, x, y, alpha, beta, st);
+        hipLaunchKernelGGL((k_spmv_strip<VT, BT, IT, RT, COMP, false>), dim3((unsigned)nblk), dim3(64 * kStripWaves),
+                           0, st, args);
     ABHSF_HIP(hipGetLastError());
     if (b.n_heavy) {
         ABHSF_REQUIRE(b.n_fix > 0 && b.n_fix < (1ll << 31), ABHSF_ERR_STATE, "fix-up table missing");
@@ -1617,13 +1641,13 @@ void launch_spmv(const DevMat &A, const Balance &B, bool coo_single, const doubl
 }
 
 template <typename VT, typename BT, typename IT, typename RT, bool COMP>
-void launch_r(int R, const DevMat &A, const Balance &Bal, bool coo_single, const double *X, int64_t ldx, double *Y,
+void launch_r(int R, const DevMat &A, const Balance &Bal, const double *X, int64_t ldx, double *Y,
               int64_t ldy, int nrhs, double alpha, double beta, hipStream_t st)
 {
     switch (R) {
     case 1:
         if (nrhs == 1 && ldx == 1 && ldy == 1)
-            launch_spmv<VT, BT, IT, RT, COMP>(A, Bal, coo_single, X, Y, alpha, beta, st);
+            launch_spmv<VT, BT, IT, RT, COMP>(A, Bal, X, Y, alpha, beta, st);
         else launch_t<VT, BT, IT, RT, 1, COMP>(A, X, ldx, Y, ldy, nrhs, alpha, beta, st);
         break;
     case 2: launch_t<VT, BT, IT, RT, 2, COMP>(A, X, ldx, Y, ldy, nrhs, alpha, beta, st); break;
@@ -1640,18 +1664,17 @@ void launch_v(const SpmvLaunch &L, const DevMat &A, int R, const double *X, int6
               int nrhs, double alpha, double beta, hipStream_t st)
 {
     const Balance &Bal = L.bal;
-    const bool cs = L.coo_single;
     const bool b16 = L.bcol_bytes == 2;
     const int s = A.s;
     if (s <= 8) {
-        if (b16) launch_r<VT, uint16_t, uint8_t, uint8_t, COMP>(R, A, Bal, cs, X, ldx, Y, ldy, nrhs, alpha, beta, st);
-        else launch_r<VT, uint32_t, uint8_t, uint8_t, COMP>(R, A, Bal, cs, X, ldx, Y, ldy, nrhs, alpha, beta, st);
+        if (b16) launch_r<VT, uint16_t, uint8_t, uint8_t, COMP>(R, A, Bal, X, ldx, Y, ldy, nrhs, alpha, beta, st);
+        else launch_r<VT, uint32_t, uint8_t, uint8_t, COMP>(R, A, Bal, X, ldx, Y, ldy, nrhs, alpha, beta, st);
     } else if (s <= 16) {
-        if (b16) launch_r<VT, uint16_t, uint8_t, uint16_t, COMP>(R, A, Bal, cs, X, ldx, Y, ldy, nrhs, alpha, beta, st);
-        else launch_r<VT, uint32_t, uint8_t, uint16_t, COMP>(R, A, Bal, cs, X, ldx, Y, ldy, nrhs, alpha, beta, st);
+        if (b16) launch_r<VT, uint16_t, uint8_t, uint16_t, COMP>(R, A, Bal, X, ldx, Y, ldy, nrhs, alpha, beta, st);
+        else launch_r<VT, uint32_t, uint8_t, uint16_t, COMP>(R, A, Bal, X, ldx, Y, ldy, nrhs, alpha, beta, st);
     } else {
-        if (b16) launch_r<VT, uint16_t, uint16_t, uint16_t, COMP>(R, A, Bal, cs, X, ldx, Y, ldy, nrhs, alpha, beta, st);
-        else launch_r<VT, uint32_t, uint16_t, uint16_t, COMP>(R, A, Bal, cs, X, ldx, Y, ldy, nrhs, alpha, beta, st);
+        if (b16) launch_r<VT, uint16_t, uint16_t, uint16_t, COMP>(R, A, Bal, X, ldx, Y, ldy, nrhs, alpha, beta, st);
+        else launch_r<VT, uint32_t, uint16_t, uint16_t, COMP>(R, A, Bal, X, ldx, Y, ldy, nrhs, alpha, beta, st);
     }
 }
 

@@ -30,10 +30,14 @@ struct Balance {
     // in (block column, strip) order.
     bool tiled = false;
     const uint32_t *coo_rng = nullptr;  // [n_light][3]
-    // the tiles' COO blocks hold 3 or more entries often enough (one in 64
-    // blocks or more) that phase B runs in most 64-block sub-chunks anyway:
-    // phase A then takes one entry per block instead of two
-    bool tile_zs1 = false;
+    // Scattered tiles over a large x (build_balance): their waves take one
+    // window of 64 entries at a time, four otherwise.  Tiles sweep x in block
+    // column order together; with more gathers in flight the fabric is busy
+    // enough that some waves fall behind, and x (beyond the L2s) is then read
+    // again for them.  block_mix s = 32, one / four windows: n = 2^22 430 /
+    // 550 us (L2 misses 27 M with four), 2.5 M 249 / 265, 2 M 202 / 198,
+    // 1 M 134 / 102 us.
+    bool tile_sweep = false;
 };
 
 #ifndef ABHSF_TILE_WORK
@@ -45,6 +49,7 @@ struct Balance {
 constexpr int kTileRows = ABHSF_TILE_ROWS;      // rows per tile at most (FP64 values)
 constexpr int kTileRowsComp = 256;              // with FP32 values (two accumulators per row)
 constexpr int64_t kTileWork = ABHSF_TILE_WORK;  // entries per tile at most
+constexpr int64_t kSweepCols = 1 << 21;         // columns above which scattered tiles sweep x in step
 
 constexpr int kXcdCount = 8;            // XCDs of an MI355X; workgroups go round-robin
 // Waves per workgroup of the single-RHS strip kernel.  Each wave runs its own
@@ -59,7 +64,6 @@ constexpr uint32_t kNoItem = 0xFFFFFFFFu;
 struct SpmvLaunch {
     int bcol_bytes;          // 2 or 4
     int val_bytes;           // 8 (f64) or 4 (f32, compensated accumulation)
-    bool coo_single = false; // COO blocks hold about one entry on average
     bool has_dense = false;  // some dense-scheme blocks (SpMM: matrix-core tiles at R >= 16)
     Balance bal;
 };

@@ -27,7 +27,8 @@ struct Storage {
     // blocks are stored in (block column, strip) order; COO z1 holds z - 1 in
     // its low coo_zb bits and the strip within the tile above them
     bool tiled = false;
-    bool tile_zs1 = false;  // tiles decode one COO entry per block in phase A (see Balance)
+    bool tile_zs1 = false;    // one in 64 or more of the tiles' COO blocks holds 3 or more entries
+    bool tile_sweep = false;  // scattered tiles over a large x (see Balance)
     int coo_zb = 16;
     DevBuf bal_coo_rng;  // tiled: [n_light][3] COO {first block, end block, first value} of each item
     // entries of the largest strip (dense blocks: positions), for the SpMM

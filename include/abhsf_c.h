@@ -110,8 +110,8 @@ typedef struct abhsf_stats {
     uint64_t index_bytes;          /* stored_bytes minus value bytes */
     double build_ms;               /* device time of the last build */
     int32_t variant;               /* ABHSF_VARIANT_* the storage was built for (AUTO resolved) */
-    int32_t tile_zs1;              /* tiled: 1 if tile COO decode takes one entry per block in its
-                                      first phase (blocks of 3+ entries are 1 in 64 or more), else 0 */
+    int32_t tile_zs1;              /* tiled: 1 if one in 64 or more of the tiles' COO blocks holds 3 or more
+                                      entries, else 0 */
     int64_t work_items;            /* single-RHS work items: light items + heavy-strip units */
     int64_t max_strip_work;        /* entries of the largest strip (dense blocks: positions); above
                                       max(4096, nnz / 4096) abhsf_spmm runs each right-hand side
