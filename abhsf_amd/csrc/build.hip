@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <numeric>
 
 namespace abhsf {
 namespace {
@@ -384,6 +385,7 @@ SpmvLaunch Storage::launch() const
     SpmvLaunch L;
     L.bcol_bytes = bcol_bytes;
     L.val_bytes = val_bytes;
+    L.coo_direct = ne[COO] < 2 * nb[COO];
     L.has_dense = nb[DENSE] > 0;
     L.bal.light = bal_light.get<uint32_t>();
     L.bal.pack = bal_pack.get<uint32_t>();
@@ -393,6 +395,7 @@ SpmvLaunch Storage::launch() const
     L.bal.part = bal_part.get<double>();
     L.bal.order = bal_order.get<uint32_t>();
     L.bal.n_light = n_light;
+    L.bal.n_lstrips = (int64_t)(bal_light.bytes() / 4);
     L.bal.n_units = n_units;
     L.bal.n_heavy = n_heavy;
     L.bal.n_slots = n_slots;
@@ -473,18 +476,18 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
     }
     ABHSF_HIP(hipStreamSynchronize(st));
     const int64_t H = 2 * unit;
-    const int64_t T = unit / 2;     // light strips are packed into items of up to T entries
-    constexpr int64_t kTiny = 128;  // ... if each holds at most kTiny entries
+    // strips per group at most: as many as leave kGroupItems items
+    const int64_t gcap = std::min<int64_t>(std::min(kGroupRows / s, kWave), std::max<int64_t>(1, M / kGroupItems));
     auto strip_work = [&](int64_t I) {
         int64_t w = 0;
         for (int x = 0; x < 4; x++) w += (int64_t)ep[x][I + 1] - ep[x][I];
         return w;
     };
-    if (panels == 1 && tile_rows <= 0) {  // nothing to split or pack: one item per strip, no tables
-        bool any = false;
+    if (panels == 1 && tile_rows <= 0) {  // nothing to split or group: one item per strip, no tables
+        bool any = gcap > 1;
         for (int64_t I = 0; I < M && !any; I++) {
             const int64_t w = strip_work(I);
-            any = w > H || (I + 1 < M && w <= kTiny && strip_work(I + 1) <= kTiny);
+            any = w > H;
         }
         if (!any) return;
     }
@@ -585,12 +588,7 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         }
         heavy.insert(heavy.end(), {(uint32_t)I, first, (uint32_t)(units.size() / 4 - first)});
     }
-    // pack runs of consecutive tiny light strips (<= kTiny entries each, one
-    // panel) into items of <= T entries and at most kPackMax strips; larger
-    // strips stay items of their own (packing those serialises work that
-    // separate wavefronts overlap: block_mix s = 16 lost 6 %)
-    constexpr size_t kPackMax = 64;
-    if (panels > 1) {  // group the light strips by panel, strip order kept inside a panel
+    if (panels > 1) {  // sort the light strips by panel, strip order kept inside a panel
         std::vector<size_t> idx(light.size());
         for (size_t i = 0; i < idx.size(); i++) idx[i] = i;
         std::stable_sort(idx.begin(), idx.end(), [&](size_t a, size_t b) { return light_panel[a] < light_panel[b]; });
@@ -623,12 +621,23 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
     }
     std::vector<uint32_t> grank, gtpos, coo_rng;
     uint64_t nrank = 0;
+    int64_t ntiles = 0;  // tiles of several strips (the first items)
+    // strips the kernel takes in groups: any up to s = 8; at s = 16 few-entry
+    // bitmap blocks (position by position in a group), from 32 on COO and CSR
+    // blocks only (its other paths take a strip at a time)
+    auto groupable = [&](uint32_t I) {
+        const bool bm = ep[BITMAP][I + 1] != ep[BITMAP][I], dn = ep[DENSE][I + 1] != ep[DENSE][I];
+        return s <= 8 || (!dn && (!bm || (s == 16 && strip_work(I) <= 128)));
+    };
     if (tile_rows > 0) {
         // items: tiles of light strips whose entries are all COO (or none), up
         // to tcap strips and kTileWork entries, gathered in strip order past
-        // strips with other groups (each of those stays an item of its own)
+        // strips with other schemes; of those, consecutive ones that can form
+        // groups do, and the rest stay items of their own
         std::vector<std::vector<uint32_t>> items;
-        int64_t open = -1, open_work = 0;
+        std::vector<char> tile;  // the item is a tile (of one strip or more)
+        int64_t open = -1, open_work = 0, gwork = 0;
+        bool gopen = false;  // the last item is a group that may take more strips
         for (size_t i = 0; i < light.size(); i++) {
             const uint32_t I = light[i];
             const int64_t cw = (int64_t)ep[COO][I + 1] - ep[COO][I];
@@ -638,7 +647,16 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
                 open_work += cw;
                 continue;
             }
+            if (!pure && gopen && groupable(I) && items.back().back() + 1 == I &&
+                (int64_t)items.back().size() < std::min(gcap, tcap) && gwork + light_work[i] <= kGroupWork) {
+                items.back().push_back(I);
+                gwork += light_work[i];
+                continue;
+            }
             items.push_back({I});
+            tile.push_back(pure);
+            gopen = !pure && groupable(I);
+            gwork = light_work[i];
             if (pure) {
                 open = (int64_t)items.size() - 1;
                 open_work = cw;
@@ -649,9 +667,9 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         // own (uniform scatter: none; R-MAT scale 22: 9 %), and from n = 2^21
         // on (x = 16 MB, four L2s) their sweep has to be kept together.
         uint64_t tile_blocks = 0, tile_ge3 = 0;
-        for (const auto &it : items) {
-            if (it.size() < 2) continue;
-            for (uint32_t I : it)
+        for (size_t q = 0; q < items.size(); q++) {
+            if (!tile[q] || items[q].size() < 2) continue;
+            for (uint32_t I : items[q])
                 for (uint64_t b = sp[COO][I]; b < sp[COO][I + 1]; b++) {
                     tile_blocks++;
                     tile_ge3 += zz[COO][b] >= 2u;
@@ -660,9 +678,19 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         tile_zs1 = tile_blocks > 0 && 64 * tile_ge3 >= tile_blocks;
         tile_sweep = tile_blocks > 0 && !tile_zs1 && n > kSweepCols;
         // tiles first: they start together and sweep x in step (their COO
-        // streams run in block-column order), the single strips fill the
+        // streams run in block-column order), the other items fill the
         // remaining slots and follow
-        std::stable_partition(items.begin(), items.end(), [](const std::vector<uint32_t> &it) { return it.size() > 1; });
+        std::vector<size_t> by_kind(items.size());
+        std::iota(by_kind.begin(), by_kind.end(), (size_t)0);
+        auto is_tile = [&](size_t q) { return tile[q] && items[q].size() > 1; };
+        std::stable_partition(by_kind.begin(), by_kind.end(), is_tile);
+        ntiles = std::count_if(by_kind.begin(), by_kind.end(), is_tile);
+        {
+            std::vector<std::vector<uint32_t>> sorted;
+            sorted.reserve(items.size());
+            for (size_t q : by_kind) sorted.push_back(std::move(items[q]));
+            items.swap(sorted);
+        }
         std::vector<uint32_t> l2;
         l2.reserve(light.size());
         for (auto &it : items) {
@@ -702,12 +730,13 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
             bs[r + 1] = bs[r] + gb[r];
             es[r + 1] = es[r] + ge[r];
         }
-        coo_rng.resize(items.size() * 3);
+        coo_rng.resize(items.size() * 4);
         for (size_t q = 0; q < items.size(); q++) {
             const size_t r = (size_t)rank_of_item[q];
-            coo_rng[3 * q] = (uint32_t)bs[r];
-            coo_rng[3 * q + 1] = (uint32_t)bs[r + 1];
-            coo_rng[3 * q + 2] = (uint32_t)es[r];
+            coo_rng[4 * q] = (uint32_t)bs[r];
+            coo_rng[4 * q + 1] = (uint32_t)bs[r + 1];
+            coo_rng[4 * q + 2] = (uint32_t)es[r];
+            coo_rng[4 * q + 3] = (int64_t)q >= ntiles;
         }
         // the COO units of a heavy strip move with the strip
         for (size_t u = 0; u < units.size() / 4; u++) {
@@ -720,16 +749,16 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         }
     } else {
         int64_t iw = 0;
-        bool tiny_item = false;  // the open item packs tiny strips
+        bool gopen = false;  // the open item may take more strips
         for (size_t i = 0; i < light.size(); i++) {
-            const bool tiny = light_work[i] <= kTiny;
-            const bool fits = !pack.empty() && tiny && tiny_item && light_panel[i] == item_panel.back() &&
-                              iw + light_work[i] <= T && i - pack.back() < kPackMax;
+            const bool gr = gcap > 1 && groupable(light[i]);
+            const bool fits = gopen && gr && light[i - 1] + 1 == light[i] && light_panel[i] == item_panel.back() &&
+                              iw + light_work[i] <= kGroupWork && (int64_t)(i - pack.back()) < gcap;
             if (!fits) {
                 pack.push_back((uint32_t)i);
                 item_panel.push_back(light_panel[i]);
                 iw = 0;
-                tiny_item = tiny;
+                gopen = gr;
             }
             iw += light_work[i];
         }
@@ -810,8 +839,6 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
             std::vector<uint32_t> uo((size_t)n_units);
             for (size_t u = 0; u < uo.size(); u++) uo[u] = (uint32_t)u;
             std::stable_sort(uo.begin(), uo.end(), [&](uint32_t a, uint32_t b) { return ucol[a] < ucol[b]; });
-            int64_t ntiles = 0;
-            while (ntiles < n_light && pack[(size_t)ntiles + 1] - pack[(size_t)ntiles] > 1) ntiles++;
             std::vector<uint32_t> ord;
             ord.reserve((size_t)(n_light + n_units + 3));
             for (int64_t i = 0; i < ntiles; i++) ord.push_back((uint32_t)i);

@@ -145,6 +145,18 @@ __device__ inline uint32_t wave_incl_scan_dpp(uint32_t v)
     return v;
 }
 
+// Inclusive prefix maximum over the 64 lanes (sources outside the row read 0).
+__device__ inline uint32_t wave_incl_max_dpp(uint32_t v)
+{
+    v = max(v, dpp_u32<DPP_ROW_SHR1>(v));
+    v = max(v, dpp_u32<DPP_ROW_SHR2>(v));
+    v = max(v, dpp_u32<DPP_ROW_SHR4>(v));
+    v = max(v, dpp_u32<DPP_ROW_SHR8>(v));
+    v = max(v, dpp_u32<DPP_ROW_BCAST15, 0xa>(v));
+    v = max(v, dpp_u32<DPP_ROW_BCAST31, 0xc>(v));
+    return v;
+}
+
 // Sum over aligned groups of G consecutive lanes (G in 1..16); every lane of
 // a group receives the group sum.
 template <int G>

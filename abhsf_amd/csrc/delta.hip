@@ -122,18 +122,6 @@ __global__ __launch_bounds__(256) void k_delta_spmv(const uint32_t *__restrict__
     }
 }
 
-// Inclusive max over the wave of values >= 0 (out-of-row DPP sources read 0).
-__device__ inline uint32_t wave_incl_max_u32(uint32_t v)
-{
-    v = max(v, dpp_u32<DPP_ROW_SHR1>(v));
-    v = max(v, dpp_u32<DPP_ROW_SHR2>(v));
-    v = max(v, dpp_u32<DPP_ROW_SHR4>(v));
-    v = max(v, dpp_u32<DPP_ROW_SHR8>(v));
-    v = max(v, dpp_u32<DPP_ROW_BCAST15, 0xa>(v));
-    v = max(v, dpp_u32<DPP_ROW_BCAST31, 0xc>(v));
-    return v;
-}
-
 // u32 delta codecs: a wavefront decodes 64 elements per step.  Deltas are
 // one coalesced u32 load; escapes (0 at any element but a chunk's first)
 // take their key from the exception list at the chunk's offset plus the
@@ -204,7 +192,7 @@ __global__ __launch_bounds__(256) void k_delta32_spmv(const uint32_t *__restrict
         const uint64_t S = wave_incl_scan_u64(esc ? 0ull : (uint64_t)d);
         uint64_t key = carry + S;
         if (mesc) {  // wave-uniform: some lane escapes in this step
-            const uint32_t last = wave_incl_max_u32(esc ? (uint32_t)lane + 1u : 0u);
+            const uint32_t last = wave_incl_max_dpp(esc ? (uint32_t)lane + 1u : 0u);
             const uint64_t b = ekey - S;  // meaningful at escape lanes
             const uint32_t src = last ? last - 1u : 0u;
             const uint32_t blo = (uint32_t)__shfl((int)(uint32_t)b, (int)src, kWaveD);

@@ -149,6 +149,29 @@ __device__ inline void group_reduce_p(double &hi, double &lo)
     }
 }
 
+// Sum (hi, lo) over aligned groups of 2^k lanes, 1 <= k <= 4 (uniform).
+template <bool COMP>
+__device__ __forceinline__ void row_reduce(int k, double &hi, double &lo)
+{
+    auto step = [&](auto ctrl_tag) {
+        constexpr int CTRL = decltype(ctrl_tag)::value;
+        const double th = dpp_f64<CTRL>(hi);
+        if constexpr (COMP) {
+            const double tl = dpp_f64<CTRL>(lo);
+            double s, e;
+            two_sum(hi, th, s, e);
+            hi = s;
+            lo += tl + e;
+        } else {
+            hi += th;
+        }
+    };
+    step(std::integral_constant<int, DPP_QUAD_XOR1>{});
+    if (k > 1) step(std::integral_constant<int, DPP_QUAD_XOR2>{});
+    if (k > 2) step(std::integral_constant<int, DPP_ROW_HALF_MIRROR>{});
+    if (k > 3) step(std::integral_constant<int, DPP_ROW_MIRROR>{});
+}
+
 template <bool COMP>
 __device__ inline void group_reduce(int P, double &hi, double &lo)
 {
@@ -171,7 +194,7 @@ static_assert(4 * 2 * 256 <= kMaskEnts, "four COO blocks per mask");
 struct WaveLds {
     uint32_t bc[kSegs];              // first column of every segment's block
     uint64_t ends[kMaskEnts / 64];   // bit t: entry t is its segment's last
-    uint8_t to[kSegs];               // tiles: the block's strip within the tile; CSR: the row
+    uint16_t to[kSegs];              // first accumulator row of the block's strip; CSR: the row
 };
 
 // Values of segments' blocks [cb, cb + nbk) of a per-block array, four
@@ -195,7 +218,7 @@ __device__ __forceinline__ void load4(const T *__restrict__ a, uint32_t cb, uint
 }
 
 // How an entry's row and column follow from its index and its segment.
-enum SegMode { SEG_COO, SEG_TILE, SEG_CSR };
+enum SegMode { SEG_COO, SEG_STRIPS, SEG_CSR };  // (one strip, several, CSR rows)
 
 // Windows of 64 consecutive entries from vp / ip on (values and in-block
 // indices: COO (lrow << k) | lcol, CSR lcol), T <= kMaskEnts entries in nseg
@@ -237,7 +260,7 @@ __device__ __forceinline__ void seg_windows(const VT *__restrict__ vp, const IT 
                 xv[u] = x[L.bc[own] + id[u]];
             } else {
                 r[u] = id[u] >> k;
-                if constexpr (MODE == SEG_TILE) r[u] += (uint32_t)L.to[own] << k;
+                if constexpr (MODE == SEG_STRIPS) r[u] += (uint32_t)L.to[own];
                 xv[u] = x[L.bc[own] + (id[u] & smask)];
             }
         }
@@ -266,6 +289,75 @@ __device__ __forceinline__ void seg_windows(const VT *__restrict__ vp, const IT 
     };
     using std::integral_constant;
     uint32_t q = 0;
+    // Full steps of long segments: a lane takes four consecutive entries and
+    // adds runs of one row as one sum.  Entries of a row lie side by side, and
+    // adds to one address are taken one lane at a time: with consecutive
+    // entries in consecutive lanes block_mix n = 217 081 s = 256 tiled (32
+    // consecutive entries a row) took 105 us with FP32 values, now 41 us;
+    // 32-row random blocks s = 128 41 -> 25 us.  COO blocks of few entries
+    // have no such runs (R-MAT scale 20 s = 256, 6 a block: 66 us, 71 this
+    // way) except where the adds return (FP32 values).
+    if (U == 4 && (COMP || MODE == SEG_CSR || T >= 16u * nseg)) {
+#pragma unroll 1
+        for (; q + (uint32_t)(4 * kWave) <= T; q += (uint32_t)(4 * kWave)) {
+            VT vw[4];
+            IT iw[4];
+            __builtin_memcpy(vw, vp + q + 4u * (uint32_t)lane, sizeof(vw));
+            __builtin_memcpy(iw, ip + q + 4u * (uint32_t)lane, sizeof(iw));
+            const uint32_t nib = (uint32_t)(L.ends[q / kWave + (uint32_t)(lane >> 4)] >> (4 * (lane & 15))) & 15u;
+            const uint32_t cnt = (uint32_t)__popc(nib), incl = wave_incl_scan_dpp(cnt);
+            const uint32_t own0 = before + incl - cnt;
+            before += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+            uint32_t r[4];
+            double xv[4], hi[4], lo[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t own = own0 + (uint32_t)__popc(nib & ((1u << i) - 1u)), id = (uint32_t)iw[i];
+                if constexpr (MODE == SEG_CSR) {
+                    r[i] = L.to[own];
+                    xv[i] = x[L.bc[own] + id];
+                } else {
+                    r[i] = id >> k;
+                    if constexpr (MODE == SEG_STRIPS) r[i] += (uint32_t)L.to[own];
+                    xv[i] = x[L.bc[own] + (id & smask)];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                hi[i] = prod<COMP>((double)vw[i], xv[i], lo[i]);
+                if (i && r[i] == r[i - 1]) {
+                    if constexpr (COMP) {
+                        double sum, err;
+                        two_sum(hi[i - 1], hi[i], sum, err);
+                        hi[i] = sum;
+                        lo[i] += lo[i - 1] + err;
+                    } else {
+                        hi[i] += hi[i - 1];
+                    }
+                }
+            }
+            auto last = [&](int i) { return i == 3 || r[i + 1] != r[i]; };
+            if constexpr (COMP) {
+                // every returning add first, then the TwoSums and the
+                // compensation adds: the returns are awaited once
+                double old[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (last(i)) old[i] = atomicAdd(&acc.hi[r[i]], hi[i]);
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (last(i)) {
+                        double sum, err;
+                        two_sum(old[i], hi[i], sum, err);
+                        atomicAdd(&acc.lo[r[i]], err + lo[i]);
+                    }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (last(i)) atomicAdd(&acc.hi[r[i]], hi[i]);
+            }
+        }
+    }
 #pragma unroll 1
     for (; q + (uint32_t)(U * kWave) <= T; q += (uint32_t)(U * kWave))
         windows(q, integral_constant<int, U>{}, std::false_type{});
@@ -286,9 +378,11 @@ __device__ __forceinline__ void seg_windows(const VT *__restrict__ vp, const IT 
 // for the row pointers, and a long row held up the wave for its whole length
 // (R-MAT scale 20 s = 256 tiled, 10 % of the entries in CSR blocks, 128 -> 64
 // us; block_mix n = 2^22 s = 128 tiled 990 -> 686 us).
+// A group of T > 1 strips from I0 on: strip I0 + t has the accumulator rows
+// from t << k on.
 template <typename VT, typename BT, typename RT, bool COMP>
 __device__ __forceinline__ void csr_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
-                                       const Acc &acc, WaveLds &L, int lane_)
+                                       const Acc &acc, WaveLds &L, int lane_, int64_t I0 = 0, int T_ = 1)
 {
     if (b0 >= b1) return;
     const MatPtr A = opaque_s(A_);
@@ -303,7 +397,9 @@ __device__ __forceinline__ void csr_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
     const uint32_t j = (4u * (uint32_t)lane) >> k, r0 = (4u * (uint32_t)lane) & ((1u << k) - 1u);
 #pragma unroll 1
     for (uint32_t cb = b0; cb < b1; cb += nb) {
-        uint32_t a[5] = {0, 0, 0, 0, 0}, bc = 0;
+        uint32_t a[5] = {0, 0, 0, 0, 0}, bc = 0, row = r0;
+        for (int t = 1; t < T_; t++)  // the block's strip
+            if (cb + j >= glob<uint32_t>(A->sptr[CSR])[I0 + t]) row = r0 + ((uint32_t)t << k);
         if (cb + j < b1) {
             const RT *__restrict__ rp = rowptr + ((uint64_t)(cb + j) * (uint64_t)((1u << k) + 1u) + r0);
             RT w[4];
@@ -330,7 +426,7 @@ __device__ __forceinline__ void csr_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
         for (int i = 0; i < 4; i++)
             if (a[i + 1] != a[i]) {
                 L.bc[o] = bc;
-                L.to[o] = (uint8_t)(r0 + (uint32_t)i);
+                L.to[o] = (uint16_t)(row + (uint32_t)i);
                 o++;
                 last[i / 2] ^= (0xFFFFu ^ (p0 + a[i + 1] - 1u)) << (16 * (i & 1));
             }
@@ -356,24 +452,68 @@ __device__ __forceinline__ void csr_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
     }
 }
 
+// Group of T consecutive strips from I0 on, scheme SC: the first block of strip
+// I0 + lane, ~0 where the strip has none (lane < T <= 64).
+template <int SC>
+__device__ __forceinline__ uint32_t group_first(MatPtr A, int64_t I0, int T, int lane)
+{
+    uint32_t first = ~0u;
+    if (lane < T) {
+        const uint32_t *sp = glob<uint32_t>(A->sptr[SC]) + I0 + lane;
+        const uint32_t f0 = sp[0], f1 = sp[1];
+        if (f1 > f0) first = f0;
+    }
+    return first;
+}
+
+// First accumulator rows (t << k) of the blocks [cb, cb + nbk) of a group, four
+// consecutive blocks per lane, into L.to: a block's strip t is the last one
+// that starts at or before it, so every strip leaves its rows at its first
+// block and a running maximum spreads them.
+__device__ __forceinline__ void group_rows(uint32_t first, uint32_t cb, uint32_t nbk, int k, WaveLds &L, int lane)
+{
+    *reinterpret_cast<uint2 *>(&L.to[4 * lane]) = make_uint2(0u, 0u);
+    wave_sync();
+    if (first > cb && first < cb + nbk) L.to[first - cb] = (uint16_t)(lane << k);
+    wave_sync();
+    const uint32_t t0 = (uint32_t)(63 - __clzll(__ballot(first <= cb))) << k;  // block cb's
+    const uint2 w = *reinterpret_cast<const uint2 *>(&L.to[4 * lane]);
+    uint32_t to[4];
+    to[0] = w.x & 0xFFFFu;
+    to[1] = max(to[0], w.x >> 16);
+    to[2] = max(to[1], w.y & 0xFFFFu);
+    to[3] = max(to[2], w.y >> 16);
+    const uint32_t up = wave_incl_max_dpp(max(to[3], t0));
+    const uint32_t left = (uint32_t)__shfl_up((int)up, 1, kWave);  // (every lane takes part)
+    const uint32_t before = lane ? left : t0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) to[i] = max(to[i], before);
+    *reinterpret_cast<uint2 *>(&L.to[4 * lane]) = make_uint2(to[0] | (to[1] << 16), to[2] | (to[3] << 16));
+}
+
 // COO group, blocks [b0, b1) with first value at offset e.  Chunks of up to
 // 256 blocks (four per lane, one prefix sum) and 2048 entries; a block is a
 // segment: it sets the bit of its last entry in the LDS mask and leaves its
 // first column in LDS.  The chunk's entries are taken in storage order, at
 // addresses known before the block metadata arrive.  A block's z1 holds z - 1
 // in its low A.zb bits and, in a tile, the block's strip t within the tile
-// above them: the tile row is (t << k) + lrow.
+// above them: the row is (t << k) + lrow.  In a group of consecutive strips
+// the blocks lie in strip order (group_rows).
 // Bound: memory latency and the x gathers.  Before, a binary search of the
 // prefix sums located every entry beyond a block's first two, which the
 // block's lane took by itself: 62 VALU instructions per 64 entries (28 now)
 // and loads that waited for the metadata.  With the CSR walk above: 27-point
 // stencil 160^3 s = 64 396 -> 262 us (4.4 TB/s), R-MAT scale 22 s = 256 tiled
 // 470 -> 354 us, scale 20 s = 64 210 -> 168 us.
-template <typename VT, typename BT, typename IT, bool COMP, bool TILE = false>
+enum CooMode { COO_STRIP, COO_TILE, COO_GROUP };
+
+template <typename VT, typename BT, typename IT, bool COMP, int MODE = COO_STRIP>
 __device__ __forceinline__ void coo_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
-                                       const Acc &acc, WaveLds &L, int lane_, bool sweep = false)
+                                       const Acc &acc, WaveLds &L, int lane_, bool sweep = false, int64_t I0 = 0,
+                                       int T_ = 1)
 {
     if (b0 >= b1) return;
+    constexpr bool TILE = MODE == COO_TILE;
     const MatPtr A = opaque_s(A_);
     const int lane = opaque_v(lane_);
     const int k = A->k, zb = TILE ? A->zb : 16;
@@ -383,18 +523,19 @@ __device__ __forceinline__ void coo_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
     const uint16_t *__restrict__ z1 = glob<uint16_t>(A->z1[COO]);
     const BT *__restrict__ bcol = glob<BT>(A->bcol[COO]);
     uint32_t *ends32 = reinterpret_cast<uint32_t *>(L.ends);
-    uint32_t cb = b0;
+    uint32_t cb = b0, first = ~0u;
+    if constexpr (MODE == COO_GROUP) first = group_first<COO>(A, I0, T_, lane);
 #pragma unroll 1
     while (cb < b1) {
         uint32_t nbk = min<uint32_t>(kSegs, b1 - cb);
         uint32_t z[4], bc[4];
         load4(z1, cb, nbk, lane, z);
         load4(bcol, cb, nbk, lane, bc);
-        uint32_t to = 0, zs = 0;
+        uint32_t to[4], zs = 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             if constexpr (TILE) {
-                to |= (z[i] >> zb) << (8 * i);
+                to[i] = (z[i] >> zb) << k;
                 z[i] &= zmask;
             }
             z[i] = 4u * (uint32_t)lane + (uint32_t)i < nbk ? z[i] + 1u : 0u;
@@ -411,7 +552,9 @@ __device__ __forceinline__ void coo_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
             nbk = min(nbk, 4u * (uint32_t)nl);
         }
         *reinterpret_cast<uint4 *>(&L.bc[4 * lane]) = make_uint4(bc[0], bc[1], bc[2], bc[3]);
-        if constexpr (TILE) *reinterpret_cast<uint32_t *>(&L.to[4 * lane]) = to;
+        if constexpr (MODE == COO_GROUP) group_rows(first, cb, nbk, k, L, lane);
+        if constexpr (TILE)
+            *reinterpret_cast<uint2 *>(&L.to[4 * lane]) = make_uint2(to[0] | (to[1] << 16), to[2] | (to[3] << 16));
         ends32[lane] = 0u;
         wave_sync();
         uint32_t p = incl - zs;
@@ -424,9 +567,10 @@ __device__ __forceinline__ void coo_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
         // one window in flight keeps the tiles' common sweep of a large x
         // together (Balance::tile_sweep)
         if (TILE && sweep)
-            seg_windows<VT, IT, COMP, SEG_TILE, 1>(val + e, idx + e, T, nbk, 0u, k, x, acc, L, lane);
+            seg_windows<VT, IT, COMP, SEG_STRIPS, 1>(val + e, idx + e, T, nbk, 0u, k, x, acc, L, lane);
         else
-            seg_windows<VT, IT, COMP, TILE ? SEG_TILE : SEG_COO, 4>(val + e, idx + e, T, nbk, 0u, k, x, acc, L, lane);
+            seg_windows<VT, IT, COMP, MODE == COO_STRIP ? SEG_COO : SEG_STRIPS, 4>(val + e, idx + e, T, nbk, 0u, k, x,
+                                                                                   acc, L, lane);
         wave_sync();
         e += T;
         cb += nbk;
@@ -548,6 +692,86 @@ __device__ __forceinline__ void bmdn_r1(MatPtr A_, int sc, uint32_t b0, uint32_t
     }
 }
 
+// Bitmap blocks of s <= 16 rows, or dense blocks of s <= 8: a lane takes one
+// position, so a wave step covers 64 consecutive positions (a quarter of a
+// 16-row block, one 8-row block, several smaller ones), four steps in flight.
+// A bitmap lane's value follows from the set bits in the lanes before it; the
+// s lanes of a row are summed with DPP and its first lane adds the sum to the
+// strip accumulator.  Block columns and, in a group of T > 1 strips from I0 on,
+// the strips' rows come from LDS, 256 blocks at a time.
+// Bound: memory latency.  One block per step, as before, was two round trips
+// per block: 2048^2 Laplacian s = 8 (a bitmap block per strip) 787 -> 118 us
+// with groups of strips, banded n = 10^6 bandwidth 40 s = 8 422 -> 186 us.
+template <typename VT, typename BT, bool COMP, int SC>
+__device__ __forceinline__ void small_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
+                                         const Acc &acc, WaveLds &L, int lane_, int64_t I0, int T_)
+{
+    if (b0 >= b1) return;
+    constexpr int U = 4;
+    const MatPtr A = opaque_s(A_);
+    const int lane = opaque_v(lane_);
+    const int k = A->k;
+    const uint32_t smask = (1u << k) - 1u, pmask = (1u << (2 * k)) - 1u;
+    const VT *__restrict__ val = glob<VT>(A->val[SC]);
+    const BT *__restrict__ bcol = glob<BT>(A->bcol[SC]);
+    const uint64_t *__restrict__ words = glob<uint64_t>(A->bm_words);
+    const int64_t n = A->n;
+    uint32_t first = ~0u;
+    if (T_ > 1) first = group_first<SC>(A, I0, T_, lane);
+#pragma unroll 1
+    for (uint32_t cb = b0; cb < b1; cb += (uint32_t)kSegs) {
+        const uint32_t nbk = min<uint32_t>(kSegs, b1 - cb);
+        uint32_t bc[4];
+        load4(bcol, cb, nbk, lane, bc);
+        *reinterpret_cast<uint4 *>(&L.bc[4 * lane]) = make_uint4(bc[0] << k, bc[1] << k, bc[2] << k, bc[3] << k);
+        if (T_ > 1) group_rows(first, cb, nbk, k, L, lane);
+        else *reinterpret_cast<uint2 *>(&L.to[4 * lane]) = make_uint2(0u, 0u);
+        wave_sync();
+        const uint32_t P = nbk << (2 * k);  // positions of the chunk
+#pragma unroll 1
+        for (uint32_t q = 0; q < P; q += (uint32_t)(U * kWave)) {
+            uint32_t bl[U], pos[U];
+            bool on[U];
+            double v[U], xv[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t pp = q + (uint32_t)(u * kWave + lane);
+                on[u] = pp < P;
+                bl[u] = min(pp, P - 1u) >> (2 * k);
+                pos[u] = pp & pmask;
+                if constexpr (SC == BITMAP) {
+                    const uint64_t w = words[((uint64_t)(cb + bl[u]) * (uint64_t)((pmask >> 6) + 1u)) + (pos[u] >> 6)];
+                    on[u] = on[u] && ((w >> (pos[u] & 63u)) & 1ull);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t c = L.bc[bl[u]] + (pos[u] & smask);
+                uint64_t off;
+                if constexpr (SC == BITMAP) {
+                    const uint64_t m = __ballot(on[u]);
+                    off = e + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                    e += (uint32_t)__popcll(m);
+                } else {
+                    on[u] = on[u] && (int64_t)c < n;  // columns past n hold stored zeros; x is not read there
+                    off = ((uint64_t)(cb + bl[u]) << (2 * k)) + pos[u];
+                }
+                v[u] = on[u] ? (double)val[off] : 0.0;
+                xv[u] = on[u] ? x[c] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                double hi, lo;
+                hi = prod<COMP>(v[u], xv[u], lo);
+                row_reduce<COMP>(k, hi, lo);
+                if ((pos[u] & smask) == 0 && q + (uint32_t)(u * kWave + lane) < P)
+                    acc_atomic<COMP>(acc, (pos[u] >> k) + L.to[bl[u]], hi, lo);
+            }
+        }
+        wave_sync();
+    }
+}
+
 // Dense group of an S-row strip (S = 16 or 32), FP64 values, coalesced: wave
 // step q reads positions q*128 + 2l, +1 of the block (1 KB contiguous); lane
 // l always has columns 2(l % L), +1 (L = S/2 lanes per row) and rows
@@ -604,27 +828,42 @@ __device__ __forceinline__ void dense_coal_r1(MatPtr A_, uint32_t b0, uint32_t b
     }
 }
 
-// Dense group of strip I: the coalesced path for FP64 16- and 32-row blocks,
-// the bitmap/dense walk otherwise.  The index types tell the block-size class
-// at compile time (u8 indices with u16 row pointers: s = 16; u16 indices:
-// s >= 32), so each kernel carries only the path it can take.
+// Dense group of a strip: the coalesced path for FP64 16- and 32-row blocks,
+// position by position for smaller ones, the bitmap/dense walk otherwise.  The
+// index types tell the block-size class at compile time (u8 indices: s <= 16,
+// with u16 row pointers s = 16; u16 indices: s >= 32), so each kernel carries
+// only the paths it can take.
 template <typename VT, typename BT, typename IT, typename RT, bool COMP>
 __device__ __forceinline__ void dense_r1(MatPtr A, uint32_t b0, uint32_t b1, const double *__restrict__ x,
-                                const Acc &acc, int lane)
+                                         const Acc &acc, WaveLds &L, int lane)
 {
+    if constexpr (sizeof(RT) == 1) {
+        small_r1<VT, BT, COMP, DENSE>(A, b0, b1, 0u, x, acc, L, lane, 0, 1);
+        return;
+    }
     if constexpr (sizeof(VT) == 8 && !COMP && sizeof(IT) == 2) {
         if (A->s == 32) {
             dense_coal_r1<BT, 32>(A, b0, b1, x, acc, lane);
             return;
         }
     }
-    if constexpr (sizeof(VT) == 8 && !COMP && sizeof(IT) == 1 && sizeof(RT) == 2) {
-        if (A->s == 16) {
-            dense_coal_r1<BT, 16>(A, b0, b1, x, acc, lane);
-            return;
-        }
+    if constexpr (sizeof(VT) == 8 && !COMP && sizeof(IT) == 1) {
+        dense_coal_r1<BT, 16>(A, b0, b1, x, acc, lane);
+        return;
     }
     bmdn_r1<VT, BT, COMP>(A, DENSE, b0, b1, 0, x, acc, lane);
+}
+
+// Bitmap group of a strip: position by position up to s = 8; a 16-row block's
+// lanes own four positions each in the lane walk and have their loads in one
+// round trip as well (27-point stencil 100^3 s = 16, FP32 values: 289 us, and
+// 508 us position by position).
+template <typename VT, typename BT, typename RT, bool COMP>
+__device__ __forceinline__ void bitmap_r1(MatPtr A, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
+                                          const Acc &acc, WaveLds &L, int lane)
+{
+    if constexpr (sizeof(RT) == 1) small_r1<VT, BT, COMP, BITMAP>(A, b0, b1, e, x, acc, L, lane, 0, 1);
+    else bmdn_r1<VT, BT, COMP>(A, BITMAP, b0, b1, e, x, acc, lane);
 }
 
 // Work items: items [0, n_light) are light items -- whole strips light[p] for
@@ -676,59 +915,75 @@ __device__ __forceinline__ void spmv_item(MatPtr A, BalPtr B, int64_t item, cons
             p1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)glob<uint32_t>(B->pack)[item + 1]);
         }
         const bool tiled = TL == 1 || (TL == 2 && B->tiled);
-        uint32_t tb0 = 0, tb1 = 0, te0 = 0;  // tiled: the item's COO blocks
+        const int T = (int)(p1 - p0);
+        const uint32_t *light = glob<uint32_t>(B->light);
+        const int64_t I = light ? (int64_t)__builtin_amdgcn_readfirstlane((int)light[p0]) : (int64_t)p0;
+        uint32_t tb0, tb1, te0, csr = 1;  // the item's COO blocks; T > 1: it has CSR blocks
         if (tiled) {
-            const uint32_t *R = glob<uint32_t>(B->coo_rng) + (uint64_t)item * 3;
+            const uint32_t *R = glob<uint32_t>(B->coo_rng) + (uint64_t)item * 4;
             tb0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[0]);
             tb1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[1]);
             te0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[2]);
-            const int T = (int)(p1 - p0);
-            if (T > 1) {
-                // a tile of strips that hold COO blocks only: one pass over
-                // them (rows (position << k) + lrow), then all rows
-                const int rows = T * s;
-                clear(rows);
-                coo_r1<VT, BT, IT, COMP, true>(A, tb0, tb1, te0, x, acc, L, lane, B->tile_sweep);
-                for (int r = lane; r < rows; r += kWave) {
-                    const int64_t gr = (int64_t)glob<uint32_t>(B->light)[p0 + (uint32_t)(r >> A->k)] * s + (r & (s - 1));
-                    if (gr < A->m) {
-                        double a = acc.hi[r];
-                        if constexpr (COMP) a += acc.lo[r];
-                        y[gr] = (beta == 0.0) ? alpha * a : alpha * a + beta * y[gr];
-                    }
-                }
+            csr = (uint32_t)__builtin_amdgcn_readfirstlane((int)R[3]);
+        } else {
+            tb0 = glob<uint32_t>(A->sptr[COO])[I];
+            tb1 = glob<uint32_t>(A->sptr[COO])[I + T];
+            te0 = glob<uint32_t>(A->eptr[COO])[I];
+        }
+        // all bounds first: one round trip (a group's strips are consecutive;
+        // a tile without CSR blocks does not use these)
+        const int64_t Ie = csr ? I + T : I;
+        const uint32_t r0 = glob<uint32_t>(A->sptr[CSR])[I], r1 = glob<uint32_t>(A->sptr[CSR])[Ie];
+        const uint32_t re = glob<uint32_t>(A->eptr[CSR])[I];
+        if (T > 1) {
+            // several strips: a tile (COO blocks only), or a group of
+            // consecutive strips; rows (position << k) + lrow
+            const int rows = T * s;
+            clear(rows);
+            if (tiled) coo_r1<VT, BT, IT, COMP, COO_TILE>(A, tb0, tb1, te0, x, acc, L, lane, B->tile_sweep);
+            else coo_r1<VT, BT, IT, COMP, COO_GROUP>(A, tb0, tb1, te0, x, acc, L, lane, false, I, T);
+            csr_r1<VT, BT, RT, COMP>(A, r0, r1, re, x, acc, L, lane, I, T);
+            if constexpr (sizeof(IT) == 1) {  // s <= 16
                 wave_sync();
-                return;
+                small_r1<VT, BT, COMP, BITMAP>(A, glob<uint32_t>(A->sptr[BITMAP])[I], glob<uint32_t>(A->sptr[BITMAP])[Ie],
+                                               glob<uint32_t>(A->eptr[BITMAP])[I], x, acc, L, lane, I, T);
             }
+            if constexpr (sizeof(RT) == 1) {  // s <= 8
+                wave_sync();
+                small_r1<VT, BT, COMP, DENSE>(A, glob<uint32_t>(A->sptr[DENSE])[I], glob<uint32_t>(A->sptr[DENSE])[Ie], 0u,
+                                              x, acc, L, lane, I, T);
+            }
+            wave_sync();
+            for (int r = lane; r < rows; r += kWave) {
+                const int64_t gr = (csr ? I + (r >> A->k) : (int64_t)light[p0 + (uint32_t)(r >> A->k)]) * s +
+                                   (r & (s - 1));
+                if (gr < A->m) {
+                    double a = acc.hi[r];
+                    if constexpr (COMP) a += acc.lo[r];
+                    y[gr] = (beta == 0.0) ? alpha * a : alpha * a + beta * y[gr];
+                }
+            }
+            wave_sync();
+            return;
         }
-#pragma unroll 1
-        for (uint32_t p = p0; p < p1; p++) {
-            const int64_t I = B->light ? (int64_t)__builtin_amdgcn_readfirstlane((int)glob<uint32_t>(B->light)[p]) : (int64_t)p;
-            // all group bounds first: one round trip
-            if (!tiled) {
-                tb0 = glob<uint32_t>(A->sptr[COO])[I];
-                tb1 = glob<uint32_t>(A->sptr[COO])[I + 1];
-                te0 = glob<uint32_t>(A->eptr[COO])[I];
-            }
-            const uint32_t r0 = glob<uint32_t>(A->sptr[CSR])[I], r1 = glob<uint32_t>(A->sptr[CSR])[I + 1], re = glob<uint32_t>(A->eptr[CSR])[I];
-            const uint32_t m0 = glob<uint32_t>(A->sptr[BITMAP])[I], m1 = glob<uint32_t>(A->sptr[BITMAP])[I + 1], me = glob<uint32_t>(A->eptr[BITMAP])[I];
-            const uint32_t d0 = glob<uint32_t>(A->sptr[DENSE])[I], d1 = glob<uint32_t>(A->sptr[DENSE])[I + 1];
-            clear(s);
-            coo_r1<VT, BT, IT, COMP>(A, tb0, tb1, te0, x, acc, L, lane);
-            csr_r1<VT, BT, RT, COMP>(A, r0, r1, re, x, acc, L, lane);
-            wave_sync();
-            bmdn_r1<VT, BT, COMP>(A, BITMAP, m0, m1, me, x, acc, lane);
-            dense_r1<VT, BT, IT, RT, COMP>(A, d0, d1, x, acc, lane);
-            wave_sync();
-            for (int r = lane; r < s; r += kWave) {
-                const int64_t gr = I * s + r;
-                if (gr >= A->m) break;
-                double a = acc.hi[r];
-                if constexpr (COMP) a += acc.lo[r];
-                y[gr] = (beta == 0.0) ? alpha * a : alpha * a + beta * y[gr];
-            }
-            wave_sync();
+        const uint32_t m0 = glob<uint32_t>(A->sptr[BITMAP])[I], m1 = glob<uint32_t>(A->sptr[BITMAP])[I + 1];
+        const uint32_t me = glob<uint32_t>(A->eptr[BITMAP])[I];
+        const uint32_t d0 = glob<uint32_t>(A->sptr[DENSE])[I], d1 = glob<uint32_t>(A->sptr[DENSE])[I + 1];
+        clear(s);
+        coo_r1<VT, BT, IT, COMP>(A, tb0, tb1, te0, x, acc, L, lane);
+        csr_r1<VT, BT, RT, COMP>(A, r0, r1, re, x, acc, L, lane);
+        wave_sync();
+        bitmap_r1<VT, BT, RT, COMP>(A, m0, m1, me, x, acc, L, lane);
+        dense_r1<VT, BT, IT, RT, COMP>(A, d0, d1, x, acc, L, lane);
+        wave_sync();
+        for (int r = lane; r < s; r += kWave) {
+            const int64_t gr = I * s + r;
+            if (gr >= A->m) break;
+            double a = acc.hi[r];
+            if constexpr (COMP) a += acc.lo[r];
+            y[gr] = (beta == 0.0) ? alpha * a : alpha * a + beta * y[gr];
         }
+        wave_sync();
     } else {
         const int64_t u = item - B->n_light;
         const uint32_t *U = glob<uint32_t>(B->units) + u * 4;
@@ -742,9 +997,9 @@ __device__ __forceinline__ void spmv_item(MatPtr A, BalPtr B, int64_t item, cons
         else if (sc == CSR)
             csr_r1<VT, BT, RT, COMP>(A, b0, b1, e0, x, acc, L, lane);
         else if (sc == BITMAP)
-            bmdn_r1<VT, BT, COMP>(A, BITMAP, b0, b1, e0, x, acc, lane);
+            bitmap_r1<VT, BT, RT, COMP>(A, b0, b1, e0, x, acc, L, lane);
         else
-            dense_r1<VT, BT, IT, RT, COMP>(A, b0, b1, x, acc, lane);
+            dense_r1<VT, BT, IT, RT, COMP>(A, b0, b1, x, acc, L, lane);
         wave_sync();
         double *part = glob_rw(B->part) + u * (size_t)s * (COMP ? 2 : 1);
         for (int r = lane; r < s; r += kWave) {
@@ -773,8 +1028,8 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_spmv_strip(StripArgs)
 {
     constexpr int kWaves = kStripWaves;
     // s rows, or a tile's (kTileRows; kTileRowsComp compensated, lo half at +256)
-    static_assert(kTileRowsComp == 256 && kTileRows >= 512, "accumulator layout");
-    __shared__ double s_acc[kWaves][kTileRows];
+    static_assert(kTileRowsComp == 256 && kGroupRows == 256 && kTileRows >= 512, "accumulator layout");
+    __shared__ double s_acc[kWaves][TILED || COMP ? kTileRows : kGroupRows];
     __shared__ __align__(16) WaveLds s_lds[kWaves];
     // the arguments, where the launch put them (the struct is the only one)
     const auto *P = (const __attribute__((address_space(4))) StripArgs *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -798,122 +1053,300 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_spmv_strip(StripArgs)
 // stored entry (i, j), i != j, y[j] += scale * a_ij * x[i], by global FP64
 // atomics (entries of a strip scatter over the column range).  FP64 values.
 // ===========================================================================
-template <typename BT, typename IT, typename RT>
-__device__ inline void trans_group(const DevMat &A, int sc, uint32_t b0, uint32_t b1, uint64_t e, int64_t I,
-                                   const double *__restrict__ x, int64_t ldx, double *y, int64_t ldy, double scale,
-                                   uint32_t *s_end, uint32_t *s_bc, int lane)
+
+// A wave takes one strip (or unit).  Its scaled x rows are kept in LDS, and the
+// products of up to kTransAcc / s blocks are summed by column in LDS before
+// they are added to y, 64 consecutive columns per wave instruction; COO blocks
+// of fewer than two entries on average (direct) are added entry by entry.
+// Bound: the global adds, which the fabric takes one request at a time.  With
+// an add for every entry (about 31 requests per wave instruction) the 27-point
+// stencil 99^3, s = 64, one triangle took 262 us for this pass, now about 70.
+constexpr int kTransAcc = 512;
+
+struct TransArgs {
+    DevMat A;
+    Balance B;
+    const double *x;
+    double *y;
+    int64_t ldx, ldy;
+    double scale;
+    int direct;
+};
+
+struct TransLds {
+    double acc[kTransAcc];  // sums by column, s per block of the chunk
+    double xs[256];         // scale * x of the strip's rows
+    WaveLds w;
+};
+
+// Sums of nb blocks from cb on to y, cleared.
+template <typename BT>
+__device__ __forceinline__ void trans_flush(const BT *__restrict__ bcol, uint32_t cb, uint32_t nb, int k, double *y,
+                                            int64_t ldy, TransLds &L, int lane)
 {
-    if (b0 >= b1) return;
-    const int s = A.s, k = A.k;
-    const uint32_t smask = (uint32_t)s - 1, ss = (uint32_t)s * (uint32_t)s;
-    const double *__restrict__ val = static_cast<const double *>(A.val[sc]);
-    const int64_t r0 = I * s;
-    auto put = [&](uint32_t lr, int64_t gc, double v) {
-        const int64_t gr = r0 + lr;
-        if (gr != gc) atomicAdd(&y[gc * ldy], scale * v * x[gr * ldx]);
-    };
-    if (sc == COO || sc == CSR) {
-        // element-parallel over chunks of 64 blocks; an entry's block by binary
-        // search over the chunk's prefix sums, its CSR row over the block's row
-        // pointers
+    wave_sync();
 #pragma unroll 1
-        for (uint32_t cb = b0; cb < b1; cb += kWave) {
-            const uint32_t jb = cb + lane;
-            const bool ok = jb < b1;
-            const uint32_t z = ok ? (uint32_t)A.z1[sc][jb] + 1u : 0u;
-            const uint32_t incl = wave_incl_scan_dpp(z);
-            const uint32_t T = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-            s_end[lane] = incl;
-            s_bc[lane] = ok ? (uint32_t)ld<BT>(A.bcol[sc], jb) : 0u;
-            wave_sync();
-            const int nbk = (int)min<uint32_t>(kWave, b1 - cb);
-#pragma unroll 1
-            for (uint32_t q = 0; q < T; q += kWave) {
-                const uint32_t t = q + lane;
-                if (t < T) {
-                    int lo = 0, hi = nbk - 1;
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if (s_end[mid] > t) hi = mid; else lo = mid + 1;
-                    }
-                    uint32_t lr, lc;
-                    if (sc == COO) {
-                        const uint32_t id = ld<IT>(A.coo_idx, e + t);
-                        lr = id >> k;
-                        lc = id & smask;
-                    } else {
-                        const uint32_t qb = t - (lo ? s_end[lo - 1] : 0u);
-                        const RT *rp = static_cast<const RT *>(A.csr_rowptr) + (uint64_t)(cb + lo) * (s + 1);
-                        int rl = 0, rh = s - 1;
-                        while (rl < rh) {
-                            const int mid = (rl + rh + 1) >> 1;
-                            if ((uint32_t)rp[mid] <= qb) rl = mid; else rh = mid - 1;
-                        }
-                        lr = (uint32_t)rl;
-                        lc = A.csr_col[e + t];
-                    }
-                    put(lr, (int64_t)s_bc[lo] * s + lc, val[e + t]);
-                }
-            }
-            e += T;
-            wave_sync();
+    for (uint32_t i = (uint32_t)lane; i < nb << k; i += kWave) {
+        const double v = L.acc[i];
+        if (v != 0.0) {
+            L.acc[i] = 0.0;
+            const int64_t gc = ((int64_t)bcol[cb + (i >> k)] << k) + (i & ((1u << k) - 1u));
+            atomicAdd(&y[gc * ldy], v);
         }
-        return;
     }
-    // bitmap / dense: one block at a time, lanes over its positions
+    wave_sync();
+}
+
+// Entries [vp, vp + T) of a chunk (COO or CSR: see seg_windows).  L.w.bc holds
+// a segment's first column (direct) or its block's first sum; L.w.to the
+// block's diagonal flag, for CSR the row with the flag in bit 15.
+template <typename IT, bool CSRM>
+__device__ __forceinline__ void trans_windows(const double *__restrict__ vp, const IT *__restrict__ ip, uint32_t T,
+                                              uint32_t nseg, uint32_t before, int k, double *y, int64_t ldy,
+                                              bool direct, TransLds &L, int lane)
+{
+    constexpr int U = 4;
+    const uint32_t smask = (1u << k) - 1u;
 #pragma unroll 1
-    for (uint32_t b = b0; b < b1; b++) {
-        const int64_t c0 = (int64_t)ld<BT>(A.bcol[sc], b) * s;
-        if (sc == DENSE) {
-            const uint64_t db = (uint64_t)b * ss;
-            for (uint32_t pos = (uint32_t)lane; pos < ss; pos += kWave) {
-                const double v = val[db + pos];
-                if (v != 0.0) put(pos >> k, c0 + (pos & smask), v);
-            }
-        } else {
-            const uint64_t *__restrict__ words = A.bm_words + (uint64_t)b * A.W;
-#pragma unroll 1
-            for (int w = 0; w < A.W; w++) {
-                const uint64_t word = words[w];
-                const uint32_t pos = (uint32_t)w * 64u + (uint32_t)lane;
-                if ((word >> lane) & 1ull)
-                    put(pos >> k, c0 + (pos & smask), val[e + __popcll(word & ((1ull << lane) - 1ull))]);
-                e += (uint64_t)__popcll(word);
+    for (uint32_t q = 0; q < T; q += (uint32_t)(U * kWave)) {
+        uint32_t id[U];
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t t = min(q + (uint32_t)(u * kWave + lane), T - 1u);
+            id[u] = ip[t];
+            v[u] = vp[t];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (q + (uint32_t)(u * kWave) >= T) break;  // uniform
+            const uint64_t m = L.w.ends[q / kWave + (uint32_t)u];
+            const uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
+            const uint32_t own = min(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, before)), nseg - 1u);
+            before += (uint32_t)__popc(lo) + (uint32_t)__popc(hi);
+            const uint32_t to = L.w.to[own];
+            const uint32_t r = CSRM ? to & 0x7FFFu : id[u] >> k, c = CSRM ? id[u] : id[u] & smask;
+            const bool diag = (CSRM ? to >> 15 : to) && r == c;
+            if (q + (uint32_t)(u * kWave + lane) < T && !diag) {
+                const double p = v[u] * L.xs[r];
+                if (direct) atomicAdd(&y[(int64_t)(L.w.bc[own] + c) * ldy], p);
+                else atomicAdd(&L.acc[L.w.bc[own] + c], p);
             }
         }
     }
 }
 
-template <typename BT, typename IT, typename RT>
-__global__ __launch_bounds__(256) void k_spmv_trans(DevMat A, Balance B, const double *__restrict__ x, int64_t ldx,
-                                                    double *y, int64_t ldy, double scale)
+template <typename BT, typename IT>
+__device__ __forceinline__ void trans_coo(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, int64_t I, double *y,
+                                          int64_t ldy, bool direct, TransLds &L, int lane)
 {
-    constexpr int kWaves = 4;
-    __shared__ uint32_t s_end[kWaves][kWave];
-    __shared__ uint32_t s_bc[kWaves][kWave];
+    if (b0 >= b1) return;
+    const MatPtr A = opaque_s(A_);
+    const int k = A->k;
+    const double *__restrict__ val = glob<double>(A->val[COO]);
+    const IT *__restrict__ idx = glob<IT>(A->coo_idx);
+    const uint16_t *__restrict__ z1 = glob<uint16_t>(A->z1[COO]);
+    const BT *__restrict__ bcol = glob<BT>(A->bcol[COO]);
+    uint32_t *ends32 = reinterpret_cast<uint32_t *>(L.w.ends);
+    const uint32_t cap = direct ? (uint32_t)kSegs : min((uint32_t)kTransAcc >> k, (uint32_t)kSegs);
+    uint32_t cb = b0;
+#pragma unroll 1
+    while (cb < b1) {
+        uint32_t nbk = min(cap, b1 - cb), z[4], bc[4], zs = 0;
+        load4(z1, cb, nbk, lane, z);
+        load4(bcol, cb, nbk, lane, bc);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            z[i] = 4u * (uint32_t)lane + (uint32_t)i < nbk ? z[i] + 1u : 0u;
+            zs += z[i];
+        }
+        const uint32_t incl = wave_incl_scan_dpp(zs);
+        uint32_t T = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        bool mine = true;
+        if (T > (uint32_t)kMaskEnts) {  // uniform: take the lanes whose blocks fit
+            mine = incl <= (uint32_t)kMaskEnts;
+            const int nl = __popcll(__ballot(mine));
+            T = (uint32_t)__builtin_amdgcn_readlane((int)incl, nl - 1);
+            nbk = min(nbk, 4u * (uint32_t)nl);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t j = 4u * (uint32_t)lane + (uint32_t)i;
+            L.w.bc[j] = direct ? bc[i] << k : j << k;
+            L.w.to[j] = (int64_t)bc[i] == I;
+        }
+        ends32[lane] = 0u;
+        wave_sync();
+        uint32_t p = incl - zs;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            p += z[i];
+            if (z[i] && mine) atomicOr(&ends32[(p - 1u) >> 5], 1u << ((p - 1u) & 31u));
+        }
+        wave_sync();
+        trans_windows<IT, false>(val + e, idx + e, T, nbk, 0u, k, y, ldy, direct, L, lane);
+        if (!direct) trans_flush(bcol, cb, nbk, k, y, ldy, L, lane);
+        wave_sync();
+        e += T;
+        cb += nbk;
+    }
+}
+
+template <typename BT, typename RT>
+__device__ __forceinline__ void trans_csr(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, int64_t I, double *y,
+                                          int64_t ldy, TransLds &L, int lane)
+{
+    if (b0 >= b1) return;
+    const MatPtr A = opaque_s(A_);
+    const int k = A->k;
+    const double *__restrict__ val = glob<double>(A->val[CSR]);
+    const uint8_t *__restrict__ ccol = glob<uint8_t>(A->csr_col);
+    const RT *__restrict__ rowptr = glob<RT>(A->csr_rowptr);
+    const BT *__restrict__ bcol = glob<BT>(A->bcol[CSR]);
+    uint32_t *ends32 = reinterpret_cast<uint32_t *>(L.w.ends);
+    const uint32_t nb = (uint32_t)kSegs >> k;  // blocks per chunk (256 rows, as csr_r1)
+    const uint32_t j = (4u * (uint32_t)lane) >> k, r0 = (4u * (uint32_t)lane) & ((1u << k) - 1u);
+#pragma unroll 1
+    for (uint32_t cb = b0; cb < b1; cb += nb) {
+        uint32_t a[5] = {0, 0, 0, 0, 0}, diag = 0;
+        if (cb + j < b1) {
+            const RT *__restrict__ rp = rowptr + ((uint64_t)(cb + j) * (uint64_t)((1u << k) + 1u) + r0);
+#pragma unroll
+            for (int i = 0; i < 5; i++) a[i] = (uint32_t)rp[i];
+            diag = (int64_t)bcol[cb + j] == I ? 0x8000u : 0u;
+        }
+        uint32_t rows = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) rows += a[i + 1] != a[i];
+        const uint32_t mine = (a[4] - a[0]) | (rows << 16);
+        const uint32_t incl = wave_incl_scan_dpp(mine);
+        const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        const uint32_t T = tot & 0xFFFFu, nseg = tot >> 16;
+        const uint32_t p0 = ((incl - mine) & 0xFFFFu) - a[0];
+        uint32_t o = (incl - mine) >> 16;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (a[i + 1] != a[i]) {
+                L.w.bc[o] = j << k;
+                L.w.to[o] = (uint16_t)(diag | (r0 + (uint32_t)i));
+                o++;
+            }
+#pragma unroll 1
+        for (uint32_t w = 0; w < T; w += (uint32_t)kMaskEnts) {
+            const uint32_t Tw = min(T - w, (uint32_t)kMaskEnts);
+            ends32[lane] = 0u;
+            wave_sync();
+            uint32_t before = 0;  // rows that end before entry w
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (a[i + 1] != a[i]) {
+                    const uint32_t last = p0 + a[i + 1] - 1u;
+                    before += last < w;
+                    if (last - w < Tw) atomicOr(&ends32[(last - w) >> 5], 1u << ((last - w) & 31u));
+                }
+            if (w) before = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan_dpp(before), kWave - 1);
+            wave_sync();
+            trans_windows<uint8_t, true>(val + (e + w), ccol + (e + w), Tw, nseg, before, k, y, ldy, false, L, lane);
+            wave_sync();
+        }
+        trans_flush(bcol, cb, min(nb, b1 - cb), k, y, ldy, L, lane);
+        e += T;
+    }
+}
+
+// Bitmap or dense blocks, one at a time, lanes over the positions.
+template <typename BT, int SC>
+__device__ __forceinline__ void trans_bmdn(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, int64_t I, double *y,
+                                           int64_t ldy, TransLds &L, int lane)
+{
+    if (b0 >= b1) return;
+    const MatPtr A = opaque_s(A_);
+    const int k = A->k;
+    const uint32_t ss = 1u << (2 * k), smask = (1u << k) - 1u, W = ss >= 64u ? ss >> 6 : 1u;
+    const double *__restrict__ val = glob<double>(A->val[SC]);
+    const uint64_t *__restrict__ words = glob<uint64_t>(A->bm_words);
+    const BT *__restrict__ bcol = glob<BT>(A->bcol[SC]);
+    const int64_t n = A->n;
+#pragma unroll 1
+    for (uint32_t b = b0; b < b1; b++) {
+        const int64_t J = (int64_t)bcol[b];
+#pragma unroll 1
+        for (uint32_t w = 0; w < W; w++) {
+            const uint32_t pos = w * 64u + (uint32_t)lane;
+            const uint32_t r = pos >> k, c = pos & smask;
+            bool on = pos < ss;
+            uint64_t off = ((uint64_t)b << (2 * k)) + pos;
+            if constexpr (SC == BITMAP) {
+                const uint64_t word = words[(uint64_t)b * W + w];
+                on = on && ((word >> lane) & 1ull);
+                off = e + __popcll(word & lanemask_lt());
+                e += (uint32_t)__popcll(word);
+            } else {
+                on = on && (J << k) + c < n;
+            }
+            if (on && !(J == I && r == c)) atomicAdd(&L.acc[c], val[off] * L.xs[r]);
+        }
+        trans_flush(bcol, b, 1u, k, y, ldy, L, lane);
+    }
+}
+
+template <typename BT, typename IT, typename RT>
+__global__ __launch_bounds__(64 * kStripWaves) void k_spmv_trans(TransArgs)
+{
+    __shared__ __align__(16) TransLds s_lds[kStripWaves];
+    const auto *P = (const __attribute__((address_space(4))) TransArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    const MatPtr A = &P->A;
+    const BalPtr B = &P->B;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t item = (int64_t)blockIdx.x * kWaves + wave;
-    if (item >= B.n_light + B.n_units) return;
-    uint32_t *se = s_end[wave], *sb = s_bc[wave];
-    if (item < B.n_light) {
-        uint32_t p0 = (uint32_t)item, p1 = (uint32_t)item + 1u;
-        if (B.pack) {
-            p0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)B.pack[item]);
-            p1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)B.pack[item + 1]);
-        }
-#pragma unroll 1
-        for (uint32_t p = p0; p < p1; p++) {
-            const int64_t I = B.light ? (int64_t)__builtin_amdgcn_readfirstlane((int)B.light[p]) : (int64_t)p;
-#pragma unroll 1
-            for (int sc = COO; sc <= DENSE; sc++)
-                trans_group<BT, IT, RT>(A, sc, A.sptr[sc][I], A.sptr[sc][I + 1],
-                                        sc == DENSE ? 0 : A.eptr[sc][I], I, x, ldx, y, ldy, scale, se, sb, lane);
-        }
+    const int64_t item = (int64_t)blockIdx.x * kStripWaves + wave;
+    if (item >= B->n_lstrips + B->n_units) return;
+    TransLds &L = s_lds[wave];
+    const int s = A->s;
+    const double *x = glob<double>(P->x);
+    double *y = glob_rw(P->y);
+    const int64_t ldy = P->ldy;
+    int64_t I;
+    uint32_t sc = 4, b0 = 0, b1 = 0, e0 = 0;  // scheme 4: a whole strip
+    if (item < B->n_lstrips) {
+        const uint32_t *light = glob<uint32_t>(B->light);
+        I = light ? (int64_t)__builtin_amdgcn_readfirstlane((int)light[item]) : item;
     } else {
-        const uint32_t *U = B.units + (item - B.n_light) * 4;
+        const uint32_t *U = glob<uint32_t>(B->units) + (item - B->n_lstrips) * 4;
         const uint32_t u0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)U[0]);
-        trans_group<BT, IT, RT>(A, (int)(u0 & 3u), U[1], U[2], U[3], (int64_t)(u0 >> 2), x, ldx, y, ldy, scale, se,
-                                sb, lane);
+        I = (int64_t)(u0 >> 2);
+        sc = u0 & 3u;
+        b0 = U[1];
+        b1 = U[2];
+        e0 = U[3];
+    }
+    for (int i = lane; i < kTransAcc; i += kWave) L.acc[i] = 0.0;
+    for (int r = lane; r < s; r += kWave) {
+        const int64_t gr = I * s + r;
+        L.xs[r] = gr < A->m ? P->scale * x[gr * P->ldx] : 0.0;
+    }
+    wave_sync();
+    // (constant scheme arguments: see spmv_item)
+    auto range = [&](int q, uint32_t &f, uint32_t &l, uint32_t &e) {
+        f = sc == 4 ? glob<uint32_t>(A->sptr[q])[I] : b0;
+        l = sc == 4 ? glob<uint32_t>(A->sptr[q])[I + 1] : b1;
+        e = sc == 4 ? glob<uint32_t>(A->eptr[q])[I] : e0;
+    };
+    uint32_t f, l, e;
+    if (sc == 4 || sc == COO) {
+        range(COO, f, l, e);
+        trans_coo<BT, IT>(A, f, l, e, I, y, ldy, P->direct != 0, L, lane);
+    }
+    if (sc == 4 || sc == CSR) {
+        range(CSR, f, l, e);
+        trans_csr<BT, RT>(A, f, l, e, I, y, ldy, L, lane);
+    }
+    if (sc == 4 || sc == BITMAP) {
+        range(BITMAP, f, l, e);
+        trans_bmdn<BT, BITMAP>(A, f, l, e, I, y, ldy, L, lane);
+    }
+    if (sc == 4 || sc == DENSE) {
+        range(DENSE, f, l, e);
+        trans_bmdn<BT, DENSE>(A, f, l, e, I, y, ldy, L, lane);
     }
 }
 
@@ -1723,16 +2156,14 @@ void spmv_transposed(const SpmvLaunch &L, const DevMat &A, int nrhs, double scal
     ABHSF_REQUIRE(L.val_bytes == 8, ABHSF_ERR_UNSUPPORTED, "symmetric storage needs FP64 values");
     if (A.M == 0) return;
     Balance b = L.bal;
-    if (!b.light && b.n_units == 0) b.n_light = A.M;
-    const int64_t nblk = (b.n_light + b.n_units + 3) / 4;
+    if (!b.light && b.n_units == 0) b.n_lstrips = A.M;
+    const int64_t nblk = (b.n_lstrips + b.n_units + kStripWaves - 1) / kStripWaves;
     ABHSF_REQUIRE(nblk < (1ll << 31), ABHSF_ERR_UNSUPPORTED, "too many strips");
     const bool b16 = L.bcol_bytes == 2;
     for (int j = 0; j < nrhs; j++) {
-        const double *x = X + j;
-        double *y = Y + j;
-#define ABHSF_TRANS(BT_, IT_, RT_)                                                                             \
-    hipLaunchKernelGGL((k_spmv_trans<BT_, IT_, RT_>), dim3((unsigned)nblk), dim3(256), 0, st, A, b, x, ldx, y, \
-                       ldy, scale)
+        const TransArgs args{A, b, X + j, Y + j, ldx, ldy, scale, L.coo_direct ? 1 : 0};
+#define ABHSF_TRANS(BT_, IT_, RT_) \
+    hipLaunchKernelGGL((k_spmv_trans<BT_, IT_, RT_>), dim3((unsigned)nblk), dim3(64 * kStripWaves), 0, st, args)
         if (A.s <= 8) {
             if (b16) ABHSF_TRANS(uint16_t, uint8_t, uint8_t); else ABHSF_TRANS(uint32_t, uint8_t, uint8_t);
         } else if (A.s <= 16) {

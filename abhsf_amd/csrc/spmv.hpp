@@ -6,9 +6,10 @@
 namespace abhsf {
 
 // Work decomposition of the single-RHS kernel: light strips are processed
-// whole, several consecutive ones per work item when they are small; heavy
-// strips are cut into units (one scheme group's block range each) whose
-// partial row sums are combined by a fix-up pass.
+// whole, groups of consecutive ones (kGroupRows rows at most) in one work item
+// where there are many of them; heavy strips are cut
+// into units (one scheme group's block range each) whose partial row sums are
+// combined by a fix-up pass.
 struct Balance {
     const uint32_t *light = nullptr;  // light strip ids (null: every strip, in order)
     const uint32_t *pack = nullptr;   // [n_light + 1] light item k = light[pack[k] .. pack[k+1])
@@ -23,13 +24,14 @@ struct Balance {
     // items are grouped by panel = XCD.
     const uint32_t *order = nullptr;  // [n_slots]
     int64_t n_light = 0, n_units = 0, n_heavy = 0, n_slots = 0, n_fix = 0;
+    int64_t n_lstrips = 0;  // length of light: the light items' strips
     // Tiled variant: light item k holds the strips light[pack[k] .. pack[k+1])
-    // (a tile of COO-only strips, or one strip), accumulated together (their
-    // rows (position << k) + lrow; kTileRows rows at most, kTileRowsComp with
-    // FP32 values); its COO blocks are coo_rng[k] = {b0, b1, first value},
-    // in (block column, strip) order.
+    // (a tile of COO-only strips, a group, or one strip), accumulated together
+    // (their rows (position << k) + lrow; kTileRows rows at most,
+    // kTileRowsComp with FP32 values); its COO blocks are coo_rng[k] = {b0,
+    // b1, first value, 0 for a tile}, in (block column, strip) order.
     bool tiled = false;
-    const uint32_t *coo_rng = nullptr;  // [n_light][3]
+    const uint32_t *coo_rng = nullptr;  // [n_light][4]
     // Scattered tiles over a large x (build_balance): their waves take one
     // window of 64 entries at a time, four otherwise.  Tiles sweep x in block
     // column order together; with more gathers in flight the fabric is busy
@@ -49,6 +51,19 @@ struct Balance {
 constexpr int kTileRows = ABHSF_TILE_ROWS;      // rows per tile at most (FP64 values)
 constexpr int kTileRowsComp = 256;              // with FP32 values (two accumulators per row)
 constexpr int64_t kTileWork = ABHSF_TILE_WORK;  // entries per tile at most
+// Groups of light strips: rows and entries at most, and the work items that are
+// left at least (kGroupItems: two waves per SIMD; a matrix with fewer than
+// twice as many strips is not grouped, its waves fill the chip by themselves).
+// A wave needs about 4 us for a strip of any small size (a chain of memory
+// round trips), so strips taken one by one, or several in turn in one wave,
+// cost their number: 2048^2 Laplacian s = 32 (160 entries a strip) 239 -> 64
+// us, s = 8 787 -> 118 us, R-MAT scale 20 s = 64 211 -> 78 us, a batch of 100
+// matrices s = 32 530 -> 289 us.  At 1024 / 4096 / 16384 items: batch 277 / 306
+// / 302 us, 100 000 rows of random 8-row blocks s = 32 8.8 / 8.1 / 8.3 us (8.2
+// here), the others alike.
+constexpr int kGroupRows = 256;
+constexpr int64_t kGroupWork = 2048;
+constexpr int64_t kGroupItems = 2048;
 constexpr int64_t kSweepCols = 1 << 21;         // columns above which scattered tiles sweep x in step
 
 constexpr int kXcdCount = 8;            // XCDs of an MI355X; workgroups go round-robin
@@ -64,6 +79,7 @@ constexpr uint32_t kNoItem = 0xFFFFFFFFu;
 struct SpmvLaunch {
     int bcol_bytes;          // 2 or 4
     int val_bytes;           // 8 (f64) or 4 (f32, compensated accumulation)
+    bool coo_direct = false; // COO blocks hold fewer than two entries on average
     bool has_dense = false;  // some dense-scheme blocks (SpMM: matrix-core tiles at R >= 16)
     Balance bal;
 };

@@ -30,7 +30,7 @@ struct Storage {
     bool tile_zs1 = false;    // one in 64 or more of the tiles' COO blocks holds 3 or more entries
     bool tile_sweep = false;  // scattered tiles over a large x (see Balance)
     int coo_zb = 16;
-    DevBuf bal_coo_rng;  // tiled: [n_light][3] COO {first block, end block, first value} of each item
+    DevBuf bal_coo_rng;  // tiled: [n_light][4] of each item (Balance::coo_rng)
     // entries of the largest strip (dense blocks: positions), for the SpMM
     // dispatch: its kernel gives each strip to one wave
     int64_t max_strip_work = 0;
@@ -41,8 +41,8 @@ struct Storage {
     DevMat view() const;
     SpmvLaunch launch() const;
     // Split strips whose work exceeds 2*unit entries into units of about
-    // `unit` entries, and pack runs of consecutive light strips into items of
-    // at most unit/2 entries (unit <= 0: neither).  With panels > 1 the block
+    // `unit` entries, and put consecutive light strips into groups where
+    // there are many strips (unit <= 0: neither).  With panels > 1 the block
     // columns are also cut into `panels` column panels of equal work: a strip
     // whose blocks span several panels is split at the panel boundaries, and
     // every work item is placed on the XCD of its panel (panels must equal the

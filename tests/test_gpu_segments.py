@@ -88,3 +88,40 @@ def test_tile_sweep_exact(gpu, n, precision):
     print(f"case sweep n={n} {precision}", flush=True)
     st = check(A, 32, "tiled", precision)
     assert not st["tile_zs1"]
+
+
+def with_integers(A, seed):
+    rng = np.random.default_rng(seed)
+    return synth.Csr(A.m, A.n, A.rowptr, A.col, (rng.integers(1, 9, A.nnz) * 1.0), A.name)
+
+
+def gaps(n, seed):
+    """Strips without entries, strips of one entry, and one long strip."""
+    rng = np.random.default_rng(seed)
+    r = np.concatenate([rng.choice(n, n // 40, replace=False), np.full(6000, n // 2), [0, n - 1]])
+    c = np.concatenate([rng.integers(0, n, n // 40), rng.choice(n, 6000, replace=False), [n - 1, 0]])
+    key = np.unique(r.astype(np.int64) * n + c)
+    return synth.from_triplets(n, n, key // n, key % n, np.ones(key.size))
+
+
+GROUPS = {  # matrices with several times 2048 strips (groups leave that many items)
+    "laplacian_301_s4": lambda: (synth.laplacian2d(301), 4),      # T up to 11, ragged last strip
+    "laplacian_700_s32": lambda: (synth.laplacian2d(700), 32),    # COO and CSR blocks, T up to 7
+    "laplacian_700_s64": lambda: (synth.laplacian2d(700), 64),
+    "rmat_17_s16": lambda: (synth.rmat(17, 8, seed=3), 16),       # bitmap strips and heavy strips between
+    "rmat_16_s2": lambda: (synth.rmat(16, 4, seed=4), 2),         # 16 strips per group
+    "gaps_s16": lambda: (gaps(100001, 5), 16),
+    "gaps_s2": lambda: (gaps(150001, 6), 2),
+}
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("variant", ["balanced", "tiled", "panel"])
+@pytest.mark.parametrize("name", list(GROUPS))
+def test_groups_exact(gpu, name, variant, precision):
+    A, s = GROUPS[name]()
+    A = with_integers(A, 1)
+    print(f"case groups {name} {variant} {precision}", flush=True)
+    st = check(A, s, variant, precision)
+    if variant != "panel":  # (panels also split every strip that spans several)
+        assert st["work_items"] < st["M"]
