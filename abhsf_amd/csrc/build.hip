@@ -81,23 +81,52 @@ __global__ void k_triangle(const int64_t *__restrict__ rp, const int32_t *__rest
     }
 }
 
-__global__ void k_rows_keys(const int64_t *__restrict__ rp, const int32_t *__restrict__ col, int64_t m, int64_t n,
-                            uint64_t nnz, int k, int jbits, uint32_t *__restrict__ rows,
-                            uint64_t *__restrict__ key, uint32_t *__restrict__ perm, uint32_t *err)
+// Row and block key of every entry, kKeyItems per thread.  The workgroup's first
+// and last entries bound its rows (two searches over all of them), and the
+// other searches go between these, in LDS: a search over all m rows per entry took
+// 316 us for R-MAT scale 20 (1.6e7 entries, 20 dependent loads each), now 185
+// us.  (One entry per thread and two full searches per 256: 284 us.)
+constexpr int kKeyItems = 16, kKeyRows = 2048;
+
+__global__ __launch_bounds__(kT) void k_rows_keys(const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                  int64_t m, int64_t n, uint64_t nnz, int k, int jbits,
+                                                  uint32_t *__restrict__ rows, uint64_t *__restrict__ key,
+                                                  uint32_t *__restrict__ perm, uint32_t *err)
 {
-    const uint64_t e = (uint64_t)blockIdx.x * kT + threadIdx.x;
-    if (e >= nnz) return;
-    int64_t lo = 0, hi = m - 1;  // last row r with rp[r] <= e
-    while (lo < hi) {
-        const int64_t mid = (lo + hi + 1) >> 1;
-        if ((uint64_t)rp[mid] <= e) lo = mid; else hi = mid - 1;
+    __shared__ int64_t bound[2];
+    __shared__ int32_t start[kKeyRows];  // first entries of the workgroup's rows, from e0
+    const uint64_t e0 = (uint64_t)blockIdx.x * (kT * kKeyItems), e1 = min(e0 + kT * kKeyItems, nnz);
+    // last r in [lo, hi] with first(r) <= at
+    auto search = [](auto first, int64_t at, int64_t lo, int64_t hi) {
+        while (lo < hi) {
+            const int64_t mid = (lo + hi + 1) >> 1;
+            if (first(mid) <= at) lo = mid; else hi = mid - 1;
+        }
+        return lo;
+    };
+    auto in_rp = [&](int64_t r) { return rp[r]; };
+    if (threadIdx.x < 2) bound[threadIdx.x] = search(in_rp, (int64_t)(threadIdx.x ? e1 - 1 : e0), 0, m - 1);
+    __syncthreads();
+    const int64_t r0 = bound[0], nr = bound[1] - r0 + 1;
+    const bool lds = nr >= 1 && nr <= kKeyRows;  // uniform
+    if (lds) {
+        for (int64_t i = threadIdx.x; i < nr; i += kT)
+            start[i] = (int32_t)max((int64_t)-1, min(rp[r0 + i] - (int64_t)e0, (int64_t)(kT * kKeyItems)));
+        __syncthreads();
     }
-    const int32_t c = col[e];
-    if (c < 0 || (int64_t)c >= n) atomicOr(err, 8u);
-    if ((int64_t)e > rp[lo] && c <= col[e - 1]) atomicOr(err, 16u);
-    rows[e] = (uint32_t)lo;
-    key[e] = ((uint64_t)((uint64_t)lo >> k) << jbits) | (uint64_t)((uint32_t)c >> k);
-    perm[e] = (uint32_t)e;
+    auto in_lds = [&](int64_t i) { return (int64_t)start[i]; };
+#pragma unroll 4
+    for (int i = 0; i < kKeyItems; i++) {
+        const uint64_t e = e0 + (uint64_t)(i * kT) + threadIdx.x;
+        if (e >= nnz) break;
+        const int64_t r = lds ? r0 + search(in_lds, (int64_t)(e - e0), 0, nr - 1) : search(in_rp, (int64_t)e, r0, bound[1]);
+        const int32_t c = col[e];
+        if (c < 0 || (int64_t)c >= n) atomicOr(err, 8u);
+        if (e > 0 && (int64_t)e > rp[r] && c <= col[e - 1]) atomicOr(err, 16u);
+        rows[e] = (uint32_t)r;
+        key[e] = ((uint64_t)((uint64_t)r >> k) << jbits) | (uint64_t)((uint32_t)c >> k);
+        perm[e] = (uint32_t)e;
+    }
 }
 
 __global__ void k_heads(const uint64_t *__restrict__ key, uint64_t nnz, uint32_t *__restrict__ flag)
@@ -318,6 +347,93 @@ __global__ void k_tile_move(uint64_t nb, const uint32_t *__restrict__ perm, cons
     }
 }
 
+// Units of heavy strip groups: workgroup g takes the blocks [b0, b1) of range
+// g = {scheme | strip << 2, b0, b1, first value} and starts a unit at every
+// block whose first value lies in another multiple of `unit` entries (counted
+// from the range's start) than the block's before it.  out null: counts[g] =
+// number of units; else the units go to out[4 * counts[g] ..] (counts then
+// holds the first unit of every range).  dense: blocks of ss positions each.
+__global__ __launch_bounds__(kT) void k_units(const uint32_t *__restrict__ ranges, Four<const uint16_t *> z1,
+                                              uint32_t ss, uint32_t unit, uint32_t *__restrict__ counts,
+                                              uint32_t *__restrict__ out)
+{
+    __shared__ uint32_t wsum[2][kT / kWave];
+    const uint32_t *R = ranges + 4 * (uint64_t)blockIdx.x;
+    const uint32_t head = R[0], x = head & 3u, b0 = R[1], b1 = R[2], e0 = R[3];
+    const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+    const uint32_t first = out ? counts[blockIdx.x] : 0u;
+    uint32_t base = 0, nu = 0, prev = 0;  // entries and units before the step; work of the block before it
+    for (uint32_t b = b0; b < b1; b += kT) {
+        const uint32_t i = b + threadIdx.x;
+        const bool ok = i < b1;
+        const uint32_t w = !ok ? 0u : x == DENSE ? ss : (uint32_t)z1.p[x][i] + 1u;
+        const uint32_t incl = wave_incl_scan_dpp(w);
+        if (lane == kWave - 1) wsum[0][wave] = incl;
+        __syncthreads();
+        uint32_t at = base + incl - w, tot = 0;
+        for (int q = 0; q < kT / kWave; q++) {
+            if (q < wave) at += wsum[0][q];
+            tot += wsum[0][q];
+        }
+        // the block before: its own start tells its unit
+        const uint32_t wl = (uint32_t)__shfl_up((int)w, 1, kWave);
+        uint32_t wp = lane ? wl : 0u;
+        if (lane == 0) {
+            if (i == b0) wp = 0;
+            else if (wave == 0) wp = prev;
+            else wp = ok ? (x == DENSE ? ss : (uint32_t)z1.p[x][i - 1] + 1u) : 0u;
+        }
+        const bool start = ok && (i == b0 || at / unit != (at - wp) / unit);
+        const uint64_t m = __ballot(start);
+        if (lane == 0) wsum[1][wave] = (uint32_t)__popcll(m);
+        __syncthreads();
+        uint32_t o = first + nu + (uint32_t)__popcll(m & lanemask_lt()), starts = 0;
+        for (int q = 0; q < kT / kWave; q++) {
+            if (q < wave) o += wsum[1][q];
+            starts += wsum[1][q];
+        }
+        if (start && out) {
+            uint32_t *U = out + 4 * (uint64_t)o;
+            U[0] = head;
+            U[1] = i;
+            U[3] = e0 + at;
+            if (i != b0) U[-2] = i;  // the unit before ends here
+        }
+        base += tot;
+        nu += starts;
+        prev = x == DENSE ? ss : (uint32_t)z1.p[x][min(b + (uint32_t)kT, b1) - 1u] + 1u;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        if (!out) counts[blockIdx.x] = nu;
+        else if (nu) out[4 * (uint64_t)(first + nu - 1u) + 2] = b1;
+    }
+}
+
+// Per strip, the COO blocks of 3 or more entries; the largest z - 1 of all.
+__global__ __launch_bounds__(kT) void k_coo_ge3(const uint32_t *__restrict__ sptr, int64_t M,
+                                                const uint16_t *__restrict__ z1, uint32_t *__restrict__ ge3,
+                                                uint32_t *__restrict__ zmax)
+{
+    const int64_t I = (int64_t)blockIdx.x * (kT / kWave) + (threadIdx.x >> 6);
+    if (I >= M) return;
+    const int lane = (int)(threadIdx.x & 63);
+    uint32_t n = 0, mx = 0;
+    for (uint32_t b = sptr[I] + (uint32_t)lane; b < sptr[I + 1]; b += kWave) {
+        n += z1[b] >= 2u;
+        mx = max(mx, (uint32_t)z1[b]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        n += (uint32_t)__shfl_xor((int)n, o, kWave);
+        mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, kWave));
+    }
+    if (lane == 0) {
+        ge3[I] = n;
+        if (mx) atomicMax(zmax, mx);
+    }
+}
+
 // First block column of every unit (units[u] = {scheme | strip << 2, b0, b1, e0}).
 __global__ void k_unit_cols(const uint32_t *__restrict__ units, int64_t n_units, Four<const void *> bcol,
                             int bcol_bytes, uint32_t *__restrict__ out)
@@ -421,27 +537,31 @@ static void tile_coo_order(Storage &S, const std::vector<uint32_t> &grp, const s
     const int bits_t = bits_for((uint64_t)std::max<int64_t>(tcap - 1, 1));
     const int key_bits = bits_for(g) + bits_bc + bits_t;
     ABHSF_REQUIRE(key_bits <= 64, ABHSF_ERR_UNSUPPORTED, "tile sort key exceeds 64 bits");
-    DevBuf dgrp((size_t)M * 4), dtpos((size_t)M * 4), keys(nb * 8), perm(nb * 4);
-    ABHSF_HIP(hipMemcpyAsync(dgrp.get(), grp.data(), dgrp.bytes(), hipMemcpyHostToDevice, st));
-    ABHSF_HIP(hipMemcpyAsync(dtpos.get(), tpos.data(), dtpos.bytes(), hipMemcpyHostToDevice, st));
+    Arena tmp(st);
+    uint32_t *dgrp = tmp.take<uint32_t>((uint64_t)M), *dtpos = tmp.take<uint32_t>((uint64_t)M);
+    uint64_t *keys = tmp.take<uint64_t>(nb);
+    uint32_t *perm = tmp.take<uint32_t>(nb);
+    ABHSF_HIP(hipMemcpyAsync(dgrp, grp.data(), (size_t)M * 4, hipMemcpyHostToDevice, st));
+    ABHSF_HIP(hipMemcpyAsync(dtpos, tpos.data(), (size_t)M * 4, hipMemcpyHostToDevice, st));
     k_tile_keys<<<grid_for(nb), kT, 0, st>>>(S.sptr[COO].get<uint32_t>(), M, nb, S.bcol[COO].get(), S.bcol_bytes,
-                                             dgrp.get<uint32_t>(), dtpos.get<uint32_t>(), bits_bc, bits_t,
-                                             keys.get<uint64_t>(), perm.get<uint32_t>());
+                                             dgrp, dtpos, bits_bc, bits_t,
+                                             keys, perm);
     ABHSF_HIP(hipGetLastError());
-    radix_sort_pairs(keys.get<uint64_t>(), perm.get<uint32_t>(), nb, key_bits, st);
-    DevBuf bc_new(S.bcol[COO].bytes()), z1_new(S.z1[COO].bytes()), znew(nb * 4), off_old(nb * 4), off_new(nb * 4);
-    k_z_count<<<grid_for(nb), kT, 0, st>>>(nb, S.z1[COO].get<uint16_t>(), off_old.get<uint32_t>());
+    radix_sort_pairs(keys, perm, nb, key_bits, st, tmp);
+    DevBuf bc_new(S.bcol[COO].bytes()), z1_new(S.z1[COO].bytes());
+    uint32_t *znew = tmp.take<uint32_t>(nb), *off_old = tmp.take<uint32_t>(nb), *off_new = tmp.take<uint32_t>(nb);
+    k_z_count<<<grid_for(nb), kT, 0, st>>>(nb, S.z1[COO].get<uint16_t>(), off_old);
     ABHSF_HIP(hipGetLastError());
-    exclusive_scan_u32(off_old.get<uint32_t>(), off_old.get<uint32_t>(), nb, nullptr, st);
-    k_tile_gather<<<grid_for(nb), kT, 0, st>>>(nb, perm.get<uint32_t>(), keys.get<uint64_t>(), bits_t, S.coo_zb,
+    exclusive_scan_u32(off_old, off_old, nb, nullptr, st, tmp);
+    k_tile_gather<<<grid_for(nb), kT, 0, st>>>(nb, perm, keys, bits_t, S.coo_zb,
                                                S.bcol[COO].get(), bc_new.get(), S.bcol_bytes,
                                                S.z1[COO].get<uint16_t>(), z1_new.get<uint16_t>(),
-                                               znew.get<uint32_t>());
+                                               znew);
     ABHSF_HIP(hipGetLastError());
-    exclusive_scan_u32(znew.get<uint32_t>(), off_new.get<uint32_t>(), nb, nullptr, st);
+    exclusive_scan_u32(znew, off_new, nb, nullptr, st, tmp);
     DevBuf v_new(S.val[COO].bytes()), i_new(S.coo_idx.bytes());
-    k_tile_move<<<grid_for(nb), kT, 0, st>>>(nb, perm.get<uint32_t>(), off_old.get<uint32_t>(),
-                                             off_new.get<uint32_t>(), znew.get<uint32_t>(), S.val[COO].get(),
+    k_tile_move<<<grid_for(nb), kT, 0, st>>>(nb, perm, off_old,
+                                             off_new, znew, S.val[COO].get(),
                                              v_new.get(), S.val_bytes, S.coo_idx.get(), i_new.get(),
                                              S.coo_idx_bytes);
     ABHSF_HIP(hipGetLastError());
@@ -491,8 +611,8 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         }
         if (!any) return;
     }
-    std::vector<uint16_t> zz[4];
-    for (int x = 0; x < 3; x++) {
+    std::vector<uint16_t> zz[4];  // (only needed for panels)
+    for (int x = 0; x < 3 && panels > 1; x++) {
         zz[x].resize(nb[x]);
         if (nb[x]) ABHSF_HIP(hipMemcpyAsync(zz[x].data(), z1[x].get(), nb[x] * 2, hipMemcpyDeviceToHost, st));
     }
@@ -536,7 +656,7 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         }
     }
     std::vector<uint32_t> light, units, heavy;
-    std::vector<uint64_t> unit_work;  // entries (dense: positions) of every unit
+    std::vector<uint32_t> ranges;  // the heavy strips' scheme groups (panels == 1)
     std::vector<uint8_t> light_panel, unit_panel;
     std::vector<int64_t> light_work;
     light.reserve((size_t)M);
@@ -558,6 +678,13 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
             light_work.push_back(w);
             continue;
         }
+        if (panels == 1) {  // cut on the device, below
+            for (int x = 0; x < 4; x++)
+                if (sp[x][I + 1] > sp[x][I])
+                    ranges.insert(ranges.end(), {(uint32_t)x | ((uint32_t)I << 2), sp[x][I], sp[x][I + 1], ep[x][I]});
+            heavy.insert(heavy.end(), {(uint32_t)I, 0u, 0u});
+            continue;
+        }
         const uint32_t first = (uint32_t)(units.size() / 4);
         for (int x = 0; x < 4; x++) {
             const uint32_t b0 = sp[x][I], b1 = sp[x][I + 1];
@@ -571,7 +698,6 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
                 if (b > ub && (p != up || acc + wz > unit)) {
                     units.insert(units.end(), {(uint32_t)x | ((uint32_t)I << 2), ub, b, (uint32_t)ue});
                     unit_panel.push_back((uint8_t)up);
-                    unit_work.push_back((uint64_t)acc);
                     ub = b;
                     ue = e;
                     acc = 0;
@@ -583,10 +709,37 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
             if (ub < b1) {
                 units.insert(units.end(), {(uint32_t)x | ((uint32_t)I << 2), ub, b1, (uint32_t)ue});
                 unit_panel.push_back((uint8_t)up);
-                unit_work.push_back((uint64_t)acc);
             }
         }
         heavy.insert(heavy.end(), {(uint32_t)I, first, (uint32_t)(units.size() / 4 - first)});
+    }
+    if (!ranges.empty()) {
+        const size_t nr = ranges.size() / 4;
+        DevBuf dr(ranges.size() * 4), dc(nr * 4);
+        ABHSF_HIP(hipMemcpyAsync(dr.get(), ranges.data(), dr.bytes(), hipMemcpyHostToDevice, st));
+        const Four<const uint16_t *> z4{{z1[0].get<uint16_t>(), z1[1].get<uint16_t>(), z1[2].get<uint16_t>(), nullptr}};
+        auto cut = [&](uint32_t *out) {
+            k_units<<<(unsigned)nr, kT, 0, st>>>(dr.get<uint32_t>(), z4, (uint32_t)ss, (uint32_t)unit,
+                                                 dc.get<uint32_t>(), out);
+            ABHSF_HIP(hipGetLastError());
+        };
+        cut(nullptr);
+        std::vector<uint32_t> first(nr + 1, 0u);
+        ABHSF_HIP(hipMemcpyAsync(first.data() + 1, dc.get(), dc.bytes(), hipMemcpyDeviceToHost, st));
+        ABHSF_HIP(hipStreamSynchronize(st));
+        for (size_t g = 0; g < nr; g++) first[g + 1] += first[g];
+        units.resize((size_t)first[nr] * 4);
+        DevBuf du(units.size() * 4);
+        ABHSF_HIP(hipMemcpyAsync(dc.get(), first.data(), dc.bytes(), hipMemcpyHostToDevice, st));
+        cut(du.get<uint32_t>());
+        ABHSF_HIP(hipMemcpyAsync(units.data(), du.get(), du.bytes(), hipMemcpyDeviceToHost, st));
+        ABHSF_HIP(hipStreamSynchronize(st));
+        size_t g = 0;
+        for (size_t h = 0; h < heavy.size() / 3; h++) {  // ranges lie in strip order
+            heavy[3 * h + 1] = first[g];
+            while (g < nr && (ranges[4 * g] >> 2) == heavy[3 * h]) g++;
+            heavy[3 * h + 2] = first[g] - heavy[3 * h + 1];
+        }
     }
     if (panels > 1) {  // sort the light strips by panel, strip order kept inside a panel
         std::vector<size_t> idx(light.size());
@@ -611,9 +764,19 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
     // 64 bits; otherwise every tile holds one strip
     int zb = 16;
     int64_t tcap = 1;
+    std::vector<uint32_t> ge3;  // COO blocks of 3 or more entries of every strip
     if (tile_rows > 0) {
         uint32_t zmax = 0;
-        for (uint64_t b = 0; b < nb[COO]; b++) zmax = std::max<uint32_t>(zmax, zz[COO][b]);
+        ge3.assign((size_t)M, 0u);
+        if (nb[COO]) {
+            DevBuf d((size_t)M * 4), mx(4);
+            ABHSF_HIP(hipMemsetAsync(mx.get(), 0, 4, st));
+            k_coo_ge3<<<grid_for((uint64_t)M * kWave), kT, 0, st>>>(sptr[COO].get<uint32_t>(), M, z1[COO].get<uint16_t>(),
+                                                                    d.get<uint32_t>(), mx.get<uint32_t>());
+            ABHSF_HIP(hipGetLastError());
+            ABHSF_HIP(hipMemcpyAsync(ge3.data(), d.get(), d.bytes(), hipMemcpyDeviceToHost, st));
+            zmax = read_dev(mx.get<uint32_t>(), st);
+        }
         zb = bits_for(zmax);
         tcap = std::min<int64_t>(tile_rows / s, zb < 16 ? (int64_t)1 << (16 - zb) : 1);
         if (bits_for((uint64_t)M) + bits_for((uint64_t)N) + bits_for((uint64_t)std::max<int64_t>(tcap - 1, 1)) > 64)
@@ -669,11 +832,10 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         uint64_t tile_blocks = 0, tile_ge3 = 0;
         for (size_t q = 0; q < items.size(); q++) {
             if (!tile[q] || items[q].size() < 2) continue;
-            for (uint32_t I : items[q])
-                for (uint64_t b = sp[COO][I]; b < sp[COO][I + 1]; b++) {
-                    tile_blocks++;
-                    tile_ge3 += zz[COO][b] >= 2u;
-                }
+            for (uint32_t I : items[q]) {
+                tile_blocks += sp[COO][I + 1] - sp[COO][I];
+                tile_ge3 += ge3[I];
+            }
         }
         tile_zs1 = tile_blocks > 0 && 64 * tile_ge3 >= tile_blocks;
         tile_sweep = tile_blocks > 0 && !tile_zs1 && n > kSweepCols;
@@ -825,8 +987,10 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         // bitmap blocks the order only loses the XCD grouping of the default
         // numbering: block_mix s = 128 1.034 -> 1.103 ms, hence the threshold)
         uint64_t coo_unit_work = 0;
-        for (int64_t u = 0; u < n_units; u++)
-            if ((units[(size_t)u * 4] & 3u) == (uint32_t)COO) coo_unit_work += unit_work[(size_t)u];
+        for (int64_t h = 0; h < n_heavy; h++) {
+            const uint32_t I = heavy[(size_t)h * 3];
+            coo_unit_work += ep[COO][I + 1] - ep[COO][I];
+        }
         if (n_units > 0 && 4 * coo_unit_work >= (uint64_t)nnz) {
             DevBuf dcol((size_t)n_units * 4);
             Four<const void *> bcp{{bcol[0].get(), bcol[1].get(), bcol[2].get(), bcol[3].get()}};
@@ -894,10 +1058,13 @@ void build_from_device_csr(Storage &S, const int64_t *rowptr, const int32_t *col
     k_check_rowptr<<<grid_for((uint64_t)m + 1), kT, 0, st>>>(rowptr, m, (int64_t)nnz, err.get<uint32_t>());
     ABHSF_HIP(hipGetLastError());
 
-    DevBuf rows(nnz * 4), key(nnz * 8), perm(nnz * 4), flag(nnz * 4), excl(nnz * 4);
+    Arena tmp(st);
+    uint32_t *rows = tmp.take<uint32_t>(nnz), *perm = tmp.take<uint32_t>(nnz), *flag = tmp.take<uint32_t>(nnz),
+             *excl = tmp.take<uint32_t>(nnz);
+    uint64_t *key = tmp.take<uint64_t>(nnz);
     if (nnz) {
-        k_rows_keys<<<grid_for(nnz), kT, 0, st>>>(rowptr, col, m, S.n, nnz, S.k, jbits, rows.get<uint32_t>(),
-                                                  key.get<uint64_t>(), perm.get<uint32_t>(), err.get<uint32_t>());
+        k_rows_keys<<<grid_for((nnz + kKeyItems - 1) / kKeyItems), kT, 0, st>>>(rowptr, col, m, S.n, nnz, S.k, jbits, rows,
+                                                  key, perm, err.get<uint32_t>());
         ABHSF_HIP(hipGetLastError());
     }
     const uint32_t ecode = read_dev(err.get<uint32_t>(), st);
@@ -906,43 +1073,44 @@ void build_from_device_csr(Storage &S, const int64_t *rowptr, const int32_t *col
                       ((ecode & 8) ? " column out of range" : "") +
                       ((ecode & 16) ? " columns not strictly increasing within a row" : "") + ")");
 
-    radix_sort_pairs(key.get<uint64_t>(), perm.get<uint32_t>(), nnz, jbits + ibits, st);
+    radix_sort_pairs(key, perm, nnz, jbits + ibits, st, tmp);
 
     uint32_t nblk = 0;
     DevBuf d_nblk(sizeof(uint32_t));
     if (nnz) {
-        k_heads<<<grid_for(nnz), kT, 0, st>>>(key.get<uint64_t>(), nnz, flag.get<uint32_t>());
+        k_heads<<<grid_for(nnz), kT, 0, st>>>(key, nnz, flag);
         ABHSF_HIP(hipGetLastError());
-        exclusive_scan_u32(flag.get<uint32_t>(), excl.get<uint32_t>(), nnz, d_nblk.get<uint32_t>(), st);
+        exclusive_scan_u32(flag, excl, nnz, d_nblk.get<uint32_t>(), st, tmp);
         nblk = read_dev(d_nblk.get<uint32_t>(), st);
     }
 
-    DevBuf bstart(((uint64_t)nblk + 1) * 4), bkey((uint64_t)nblk * 8), sch((uint64_t)nblk);
-    DevBuf cnt[4], ecnt[4];
+    uint32_t *bstart = tmp.take<uint32_t>((uint64_t)nblk + 1), *cnt[4], *ecnt[4];
+    uint64_t *bkey = tmp.take<uint64_t>(nblk);
+    uint8_t *sch = tmp.take<uint8_t>(nblk);
     for (int x = 0; x < 4; x++) {
-        cnt[x].alloc((uint64_t)nblk * 4);
-        ecnt[x].alloc((uint64_t)nblk * 4);
+        cnt[x] = tmp.take<uint32_t>(nblk);
+        ecnt[x] = tmp.take<uint32_t>(nblk);
     }
     DevBuf totals(6 * sizeof(unsigned long long));
     ABHSF_HIP(hipMemsetAsync(totals.get(), 0, totals.bytes(), st));
     unsigned long long htot[6] = {0, 0, 0, 0, 0, 0};
     const uint64_t nwg = grid_for(nblk);
-    DevBuf partial(6 * nwg * sizeof(unsigned long long));
+    uint64_t *partial = tmp.take<uint64_t>(6 * nwg);
     if (nnz) {
-        k_block_starts<<<grid_for(nnz), kT, 0, st>>>(key.get<uint64_t>(), flag.get<uint32_t>(),
-                                                     excl.get<uint32_t>(), nnz, nblk, bstart.get<uint32_t>(),
-                                                     bkey.get<uint64_t>());
+        k_block_starts<<<grid_for(nnz), kT, 0, st>>>(key, flag,
+                                                     excl, nnz, nblk, bstart,
+                                                     bkey);
         ABHSF_HIP(hipGetLastError());
         Four<uint32_t *> c4, e4;
-        for (int x = 0; x < 4; x++) { c4.p[x] = cnt[x].get<uint32_t>(); e4.p[x] = ecnt[x].get<uint32_t>(); }
+        for (int x = 0; x < 4; x++) { c4.p[x] = cnt[x]; e4.p[x] = ecnt[x]; }
         const uint64_t hdr = ceil_log2_u64((uint64_t)M) + ceil_log2_u64((uint64_t)S.N) + 2;  // test.cpp:49
-        k_block_scheme<<<(unsigned)nwg, kT, 0, st>>>(bstart.get<uint32_t>(), nblk, S.s, S.policy, S.cost_b,
-                                                     S.is_binary, hdr, sch.get<uint8_t>(), c4, e4,
-                                                     partial.get<unsigned long long>());
+        k_block_scheme<<<(unsigned)nwg, kT, 0, st>>>(bstart, nblk, S.s, S.policy, S.cost_b,
+                                                     S.is_binary, hdr, sch, c4, e4,
+                                                     reinterpret_cast<unsigned long long *>(partial));
         ABHSF_HIP(hipGetLastError());
         for (int q = 0; q < 6; q++) {
-            uint64_t *pq = partial.get<uint64_t>() + (uint64_t)q * nwg;
-            exclusive_scan_u64(pq, pq, nwg, totals.get<uint64_t>() + q, st);
+            uint64_t *pq = partial + (uint64_t)q * nwg;
+            exclusive_scan_u64(pq, pq, nwg, totals.get<uint64_t>() + q, st, tmp);
         }
         ABHSF_HIP(hipMemcpyAsync(htot, totals.get(), sizeof(htot), hipMemcpyDeviceToHost, st));
         ABHSF_HIP(hipStreamSynchronize(st));
@@ -957,8 +1125,8 @@ void build_from_device_csr(Storage &S, const int64_t *rowptr, const int32_t *col
     DevBuf tot4(8 * sizeof(uint32_t));
     ABHSF_HIP(hipMemsetAsync(tot4.get(), 0, tot4.bytes(), st));
     for (int x = 0; x < 4; x++) {
-        exclusive_scan_u32(cnt[x].get<uint32_t>(), cnt[x].get<uint32_t>(), nblk, tot4.get<uint32_t>() + x, st);
-        exclusive_scan_u32(ecnt[x].get<uint32_t>(), ecnt[x].get<uint32_t>(), nblk, tot4.get<uint32_t>() + 4 + x, st);
+        exclusive_scan_u32(cnt[x], cnt[x], nblk, tot4.get<uint32_t>() + x, st, tmp);
+        exclusive_scan_u32(ecnt[x], ecnt[x], nblk, tot4.get<uint32_t>() + 4 + x, st, tmp);
     }
     uint32_t h4[8];
     ABHSF_HIP(hipMemcpyAsync(h4, tot4.get(), sizeof(h4), hipMemcpyDeviceToHost, st));
@@ -990,8 +1158,8 @@ void build_from_device_csr(Storage &S, const int64_t *rowptr, const int32_t *col
     Four<void *> bc;
     Four<uint16_t *> zz;
     for (int x = 0; x < 4; x++) {
-        ord.p[x] = cnt[x].get<uint32_t>();
-        eoff.p[x] = ecnt[x].get<uint32_t>();
+        ord.p[x] = cnt[x];
+        eoff.p[x] = ecnt[x];
         nbx.p[x] = (uint32_t)S.nb[x];
         nex.p[x] = (uint32_t)S.ne[x];
         sp.p[x] = S.sptr[x].get<uint32_t>();
@@ -1005,10 +1173,10 @@ void build_from_device_csr(Storage &S, const int64_t *rowptr, const int32_t *col
             ABHSF_HIP(hipMemsetAsync(S.eptr[x].get(), 0, S.eptr[x].bytes(), st));
         }
     } else {
-        k_strip_ptrs<<<grid_for(nblk), kT, 0, st>>>(bkey.get<uint64_t>(), nblk, jbits, M, ord, eoff, nbx, nex, sp, ep);
+        k_strip_ptrs<<<grid_for(nblk), kT, 0, st>>>(bkey, nblk, jbits, M, ord, eoff, nbx, nex, sp, ep);
         ABHSF_HIP(hipGetLastError());
         const uint64_t jmask = (jbits >= 64) ? ~0ull : ((1ull << jbits) - 1);
-        k_block_meta<<<grid_for(nblk), kT, 0, st>>>(bkey.get<uint64_t>(), bstart.get<uint32_t>(), sch.get<uint8_t>(),
+        k_block_meta<<<grid_for(nblk), kT, 0, st>>>(bkey, bstart, sch,
                                                     nblk, jmask, S.bcol_bytes, ord, bc, zz);
         ABHSF_HIP(hipGetLastError());
         EmitOut out;
@@ -1021,8 +1189,8 @@ void build_from_device_csr(Storage &S, const int64_t *rowptr, const int32_t *col
         out.csr_rp_bytes = S.csr_rp_bytes;
         out.val_bytes = vb;
         out.W = S.W;
-        k_emit<<<grid_for(nnz), kT, 0, st>>>(flag.get<uint32_t>(), excl.get<uint32_t>(), bstart.get<uint32_t>(),
-                                             sch.get<uint8_t>(), perm.get<uint32_t>(), rows.get<uint32_t>(), col, val,
+        k_emit<<<grid_for(nnz), kT, 0, st>>>(flag, excl, bstart,
+                                             sch, perm, rows, col, val,
                                              nnz, S.s, S.k, ord, eoff, out);
         ABHSF_HIP(hipGetLastError());
     }

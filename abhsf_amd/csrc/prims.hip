@@ -5,8 +5,23 @@
 // (preprocessing/test.cpp:237-368).
 #include "prims.hpp"
 
+#include <algorithm>
+#include <mutex>
+#include <utility>
+
 namespace abhsf {
 namespace {
+
+// Scratch kept between operations, per device.
+struct Kept {
+    std::mutex m;
+    std::vector<std::pair<int, DevBuf>> bufs;
+};
+Kept &kept()
+{
+    static Kept *k = new Kept;  // (not destroyed: the HIP runtime may end before static objects do)
+    return *k;
+}
 
 constexpr int kThreads = 256;
 constexpr int kItems = 8;
@@ -98,7 +113,7 @@ __global__ __launch_bounds__(kThreads) void k_tile_scan(const T *in, T *out, uin
 }
 
 template <typename T>
-void exclusive_scan_impl(const T *in, T *out, uint64_t n, T *total, hipStream_t st, std::vector<DevBuf> &keep)
+void exclusive_scan_impl(const T *in, T *out, uint64_t n, T *total, hipStream_t st, Arena &tmp)
 {
     if (n == 0) {
         if (total) ABHSF_HIP(hipMemsetAsync(total, 0, sizeof(T), st));
@@ -110,11 +125,10 @@ void exclusive_scan_impl(const T *in, T *out, uint64_t n, T *total, hipStream_t 
         ABHSF_HIP(hipGetLastError());
         return;
     }
-    keep.emplace_back(ntiles * sizeof(T));
-    T *sums = keep.back().get<T>();
+    T *sums = tmp.take<T>(ntiles);
     k_tile_reduce<T><<<(unsigned)ntiles, kThreads, 0, st>>>(in, n, sums);
     ABHSF_HIP(hipGetLastError());
-    exclusive_scan_impl<T>(sums, sums, ntiles, total, st, keep);
+    exclusive_scan_impl<T>(sums, sums, ntiles, total, st, tmp);
     k_tile_scan<T><<<(unsigned)ntiles, kThreads, 0, st>>>(in, out, n, sums, nullptr);
     ABHSF_HIP(hipGetLastError());
 }
@@ -191,36 +205,106 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const uint64_t *__re
 
 }  // namespace
 
-void exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint32_t *total, hipStream_t st)
+bool scratch_trim()
 {
-    std::vector<DevBuf> keep;
-    exclusive_scan_impl<uint32_t>(in, out, n, total, st, keep);
-    if (!keep.empty()) ABHSF_HIP(hipStreamSynchronize(st));
+    std::vector<std::pair<int, DevBuf>> out;
+    {
+        std::lock_guard<std::mutex> l(kept().m);
+        out.swap(kept().bufs);
+    }
+    return !out.empty();  // freed here
 }
 
-void exclusive_scan_u64(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total, hipStream_t st)
+Arena::Arena(hipStream_t st) : st_(st)
 {
-    std::vector<DevBuf> keep;
-    exclusive_scan_impl<uint64_t>(in, out, n, total, st, keep);
-    if (!keep.empty()) ABHSF_HIP(hipStreamSynchronize(st));
+    ABHSF_HIP(hipGetDevice(&device_));
+    std::lock_guard<std::mutex> l(kept().m);
+    auto &b = kept().bufs;
+    for (size_t i = 0; i < b.size();) {
+        if (b[i].first != device_) {
+            i++;
+            continue;
+        }
+        kept_.push_back(std::move(b[i].second));
+        b[i] = std::move(b.back());
+        b.pop_back();
+    }
 }
 
-void radix_sort_pairs(uint64_t *keys, uint32_t *vals, uint64_t n, int key_bits, hipStream_t st)
+Arena::~Arena()
+{
+    // nothing on the stream uses the buffers any more; after an error they go
+    // back to the runtime
+    if (hipStreamSynchronize(st_) != hipSuccess) return;
+    try {
+        std::lock_guard<std::mutex> l(kept().m);
+        size_t total = 0;
+        for (const auto &b : kept().bufs)
+            if (b.first == device_) total += b.second.bytes();
+        for (auto &b : used_)
+            if (total + b.bytes() <= kScratchKeep) {
+                total += b.bytes();
+                kept().bufs.emplace_back(device_, std::move(b));
+            }
+    } catch (...) {  // out of host memory: what is left is freed
+    }
+}
+
+void *Arena::fresh(size_t bytes)
+{
+    size_t best = kept_.size();
+    for (size_t i = 0; i < kept_.size(); i++)
+        if (kept_[i].bytes() >= bytes && kept_[i].bytes() <= 2 * bytes &&
+            (best == kept_.size() || kept_[i].bytes() < kept_[best].bytes()))
+            best = i;
+    if (best < kept_.size()) {
+        used_.push_back(std::move(kept_[best]));
+        kept_.erase(kept_.begin() + (std::ptrdiff_t)best);
+    } else {
+        DevBuf b(bytes);
+        used_.push_back(std::move(b));
+    }
+    return used_.back().get();
+}
+
+void *Arena::take_bytes(size_t bytes)
+{
+    bytes = (bytes + 255) & ~(size_t)255;
+    if (bytes == 0) return nullptr;
+    if (bytes > kChunk) return fresh(bytes);
+    if (!chunk_ || at_ + bytes > kChunk) {
+        chunk_ = static_cast<char *>(fresh(kChunk));
+        at_ = 0;
+    }
+    void *p = chunk_ + at_;
+    at_ += bytes;
+    return p;
+}
+
+void exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint32_t *total, hipStream_t st, Arena &tmp)
+{
+    exclusive_scan_impl<uint32_t>(in, out, n, total, st, tmp);
+}
+
+void exclusive_scan_u64(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total, hipStream_t st, Arena &tmp)
+{
+    exclusive_scan_impl<uint64_t>(in, out, n, total, st, tmp);
+}
+
+void radix_sort_pairs(uint64_t *keys, uint32_t *vals, uint64_t n, int key_bits, hipStream_t st, Arena &tmp)
 {
     if (n < 2 || key_bits <= 0) return;
     ABHSF_REQUIRE(n < (1ull << 32), ABHSF_ERR_UNSUPPORTED, "radix sort limited to 2^32 elements");
     const uint64_t ntiles = (n + kTile - 1) / kTile;
     ABHSF_REQUIRE(ntiles * kRadix < (1ull << 32), ABHSF_ERR_UNSUPPORTED, "radix histogram too large");
-    DevBuf k2(n * sizeof(uint64_t)), v2(n * sizeof(uint32_t)), hist(ntiles * kRadix * sizeof(uint32_t));
-    uint64_t *ka = keys, *kb = k2.get<uint64_t>();
-    uint32_t *va = vals, *vb = v2.get<uint32_t>();
-    std::vector<DevBuf> keep;
+    uint64_t *ka = keys, *kb = tmp.take<uint64_t>(n);
+    uint32_t *va = vals, *vb = tmp.take<uint32_t>(n);
+    uint32_t *hist = tmp.take<uint32_t>(ntiles * kRadix);
     for (int shift = 0; shift < key_bits; shift += kRadixBits) {
-        k_radix_hist<<<(unsigned)ntiles, kThreads, 0, st>>>(ka, n, shift, hist.get<uint32_t>(), (uint32_t)ntiles);
+        k_radix_hist<<<(unsigned)ntiles, kThreads, 0, st>>>(ka, n, shift, hist, (uint32_t)ntiles);
         ABHSF_HIP(hipGetLastError());
-        exclusive_scan_impl<uint32_t>(hist.get<uint32_t>(), hist.get<uint32_t>(), ntiles * kRadix, nullptr, st, keep);
-        k_radix_scatter<<<(unsigned)ntiles, kThreads, 0, st>>>(ka, va, kb, vb, n, shift, hist.get<uint32_t>(),
-                                                                (uint32_t)ntiles);
+        exclusive_scan_impl<uint32_t>(hist, hist, ntiles * kRadix, nullptr, st, tmp);
+        k_radix_scatter<<<(unsigned)ntiles, kThreads, 0, st>>>(ka, va, kb, vb, n, shift, hist, (uint32_t)ntiles);
         ABHSF_HIP(hipGetLastError());
         std::swap(ka, kb);
         std::swap(va, vb);
@@ -229,7 +313,6 @@ void radix_sort_pairs(uint64_t *keys, uint32_t *vals, uint64_t n, int key_bits, 
         ABHSF_HIP(hipMemcpyAsync(keys, ka, n * sizeof(uint64_t), hipMemcpyDeviceToDevice, st));
         ABHSF_HIP(hipMemcpyAsync(vals, va, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
     }
-    ABHSF_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace abhsf

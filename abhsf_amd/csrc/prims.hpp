@@ -7,6 +7,9 @@
 
 namespace abhsf {
 
+// Frees the scratch kept between operations (Arena); false if there was none.
+bool scratch_trim();
+
 // RAII device buffer.
 class DevBuf {
   public:
@@ -27,6 +30,7 @@ class DevBuf {
         n_ = bytes;
         if (bytes == 0) return;
         hipError_t e = hipMalloc(&p_, bytes);
+        if (e != hipSuccess && scratch_trim()) e = hipMalloc(&p_, bytes);
         if (e != hipSuccess) {
             p_ = nullptr;
             n_ = 0;
@@ -49,13 +53,47 @@ class DevBuf {
     size_t n_ = 0;
 };
 
+// Device scratch of one operation on a stream, handed out piece by piece.  A
+// conversion needs some thirty pieces, about 36 bytes an entry in all, and
+// allocating and freeing them every time cost more than its kernels: a free
+// waits for the device, and freed memory is cleared before it is given out
+// again (converting R-MAT scale 20, 0.9 GB of scratch, again and again: 12 ms
+// at first, 28 ms once the clearing lags behind).  Small pieces share chunks;
+// the buffers of the last operation stay for the next one: at most
+// kScratchKeep bytes per device, no others than that operation used, and none
+// if an allocation fails.  An Arena owns what it took until it is destroyed,
+// after the stream has finished, so operations of several threads or streams
+// never share a buffer.  Pieces are 256-byte aligned.
+constexpr size_t kScratchKeep = (size_t)1 << 30;
+
+class Arena {
+  public:
+    explicit Arena(hipStream_t st);
+    ~Arena();
+    Arena(const Arena &) = delete;
+    Arena &operator=(const Arena &) = delete;
+    void *take_bytes(size_t bytes);
+    template <typename T>
+    T *take(uint64_t n) { return static_cast<T *>(take_bytes((size_t)n * sizeof(T))); }
+
+  private:
+    static constexpr size_t kChunk = (size_t)16 << 20;
+    void *fresh(size_t bytes);  // a kept buffer that fits, or a new one
+    std::vector<DevBuf> kept_, used_;
+    char *chunk_ = nullptr;
+    size_t at_ = 0;
+    int device_ = 0;
+    hipStream_t st_;
+};
+
 // Exclusive scan out[i] = sum_{j<i} in[j]; out may alias in.  If total is
-// non-null the sum of all n inputs is written there (device pointer).
-void exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint32_t *total, hipStream_t st);
-void exclusive_scan_u64(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total, hipStream_t st);
+// non-null the sum of all n inputs is written there (device pointer).  The
+// scratch stays in `tmp`; the calls only enqueue.
+void exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint32_t *total, hipStream_t st, Arena &tmp);
+void exclusive_scan_u64(const uint64_t *in, uint64_t *out, uint64_t n, uint64_t *total, hipStream_t st, Arena &tmp);
 
 // Stable LSD radix sort of (key, value) pairs by the low key_bits of key.
-// keys/vals are sorted in place (scratch of the same sizes is allocated).
-void radix_sort_pairs(uint64_t *keys, uint32_t *vals, uint64_t n, int key_bits, hipStream_t st);
+// keys/vals are sorted in place (scratch of the same sizes comes from tmp).
+void radix_sort_pairs(uint64_t *keys, uint32_t *vals, uint64_t n, int key_bits, hipStream_t st, Arena &tmp);
 
 }  // namespace abhsf

@@ -116,26 +116,30 @@ extern "C" abhsf_status abhsf_block_hist_impl(const int64_t *rowptr, const int32
             rp = drp.get<int64_t>();
             cl = dc.get<int32_t>();
         }
-        DevBuf cnt((uint64_t)m * 4), tot(4);
-        k_sample_counts<<<grid_for((uint64_t)m), kT, 0, st>>>(rp, m, kr, strip_stride, cnt.get<uint32_t>());
+        Arena tmp(st);
+        DevBuf tot(4);
+        uint32_t *cnt = tmp.take<uint32_t>((uint64_t)m);
+        k_sample_counts<<<grid_for((uint64_t)m), kT, 0, st>>>(rp, m, kr, strip_stride, cnt);
         ABHSF_HIP(hipGetLastError());
-        exclusive_scan_u32(cnt.get<uint32_t>(), cnt.get<uint32_t>(), (uint64_t)m, tot.get<uint32_t>(), st);
+        exclusive_scan_u32(cnt, cnt, (uint64_t)m, tot.get<uint32_t>(), st, tmp);
         uint32_t ns = 0;
         ABHSF_HIP(hipMemcpyAsync(&ns, tot.get(), 4, hipMemcpyDeviceToHost, st));
         ABHSF_HIP(hipStreamSynchronize(st));
         if (sampled_nnz) *sampled_nnz = ns;
-        DevBuf key((uint64_t)ns * 8), pay((uint64_t)ns * 4), dh((uint64_t)hist_cap * 8), dnb(8);
+        DevBuf dh((uint64_t)hist_cap * 8), dnb(8);
+        uint64_t *key = tmp.take<uint64_t>(ns);
+        uint32_t *pay = tmp.take<uint32_t>(ns);
         ABHSF_HIP(hipMemsetAsync(dh.get(), 0, dh.bytes(), st));
         ABHSF_HIP(hipMemsetAsync(dnb.get(), 0, 8, st));
         const int jbits = bits_for((uint64_t)((n - 1) >> ks));
         const int ibits = bits_for((uint64_t)((m - 1) >> kr));
         if (ns) {
             k_sample_keys<<<grid_for((uint64_t)nnz), kT, 0, st>>>(rp, cl, m, (uint64_t)nnz, kr, ks, jbits,
-                                                                  strip_stride, cnt.get<uint32_t>(),
-                                                                  key.get<uint64_t>(), pay.get<uint32_t>());
+                                                                  strip_stride, cnt,
+                                                                  key, pay);
             ABHSF_HIP(hipGetLastError());
-            radix_sort_pairs(key.get<uint64_t>(), pay.get<uint32_t>(), ns, jbits + ibits, st);
-            k_runs_hist<<<grid_for(ns), kT, 0, st>>>(key.get<uint64_t>(), ns, dh.get<unsigned long long>(),
+            radix_sort_pairs(key, pay, ns, jbits + ibits, st, tmp);
+            k_runs_hist<<<grid_for(ns), kT, 0, st>>>(key, ns, dh.get<unsigned long long>(),
                                                       (uint64_t)hist_cap, dnb.get<unsigned long long>());
             ABHSF_HIP(hipGetLastError());
         }
