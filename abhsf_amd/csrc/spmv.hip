@@ -1284,7 +1284,11 @@ __device__ __forceinline__ void trans_bmdn(MatPtr A_, uint32_t b0, uint32_t b1, 
             } else {
                 on = on && (J << k) + c < n;
             }
-            if (on && !(J == I && r == c)) atomicAdd(&L.acc[c], val[off] * L.xs[r]);
+            const double v = on ? val[off] : 0.0;
+            // zeros fill a dense block where it has no entry: not a product
+            // (x there may be infinite)
+            if (SC == DENSE) on = on && v != 0.0;
+            if (on && !(J == I && r == c)) atomicAdd(&L.acc[c], v * L.xs[r]);
         }
         trans_flush(bcol, b, 1u, k, y, ldy, L, lane);
     }
