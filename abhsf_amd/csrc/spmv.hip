@@ -1054,8 +1054,8 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_spmv_strip(StripArgs)
 // atomics (entries of a strip scatter over the column range).  FP64 values.
 // ===========================================================================
 
-// A wave takes one strip (or unit).  Its scaled x rows are kept in LDS, and the
-// products of up to kTransAcc / s blocks are summed by column in LDS before
+// A wave takes one strip (or unit).  Its x rows are kept in LDS, and the
+// products (scale v) x (scale x may leave the range where scale v does not) of up to kTransAcc / s blocks are summed by column in LDS before
 // they are added to y, 64 consecutive columns per wave instruction; COO blocks
 // of fewer than two entries on average (direct) are added entry by entry.
 // Bound: the global adds, which the fabric takes one request at a time.  With
@@ -1075,7 +1075,7 @@ struct TransArgs {
 
 struct TransLds {
     double acc[kTransAcc];  // sums by column, s per block of the chunk
-    double xs[256];         // scale * x of the strip's rows
+    double xs[256];         // x of the strip's rows
     WaveLds w;
 };
 
@@ -1103,7 +1103,7 @@ __device__ __forceinline__ void trans_flush(const BT *__restrict__ bcol, uint32_
 template <typename IT, bool CSRM>
 __device__ __forceinline__ void trans_windows(const double *__restrict__ vp, const IT *__restrict__ ip, uint32_t T,
                                               uint32_t nseg, uint32_t before, int k, double *y, int64_t ldy,
-                                              bool direct, TransLds &L, int lane)
+                                              double scale, bool direct, TransLds &L, int lane)
 {
     constexpr int U = 4;
     const uint32_t smask = (1u << k) - 1u;
@@ -1128,7 +1128,7 @@ __device__ __forceinline__ void trans_windows(const double *__restrict__ vp, con
             const uint32_t r = CSRM ? to & 0x7FFFu : id[u] >> k, c = CSRM ? id[u] : id[u] & smask;
             const bool diag = (CSRM ? to >> 15 : to) && r == c;
             if (q + (uint32_t)(u * kWave + lane) < T && !diag) {
-                const double p = v[u] * L.xs[r];
+                const double p = (scale * v[u]) * L.xs[r];
                 if (direct) atomicAdd(&y[(int64_t)(L.w.bc[own] + c) * ldy], p);
                 else atomicAdd(&L.acc[L.w.bc[own] + c], p);
             }
@@ -1138,7 +1138,7 @@ __device__ __forceinline__ void trans_windows(const double *__restrict__ vp, con
 
 template <typename BT, typename IT>
 __device__ __forceinline__ void trans_coo(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, int64_t I, double *y,
-                                          int64_t ldy, bool direct, TransLds &L, int lane)
+                                          int64_t ldy, double scale, bool direct, TransLds &L, int lane)
 {
     if (b0 >= b1) return;
     const MatPtr A = opaque_s(A_);
@@ -1184,7 +1184,7 @@ __device__ __forceinline__ void trans_coo(MatPtr A_, uint32_t b0, uint32_t b1, u
             if (z[i] && mine) atomicOr(&ends32[(p - 1u) >> 5], 1u << ((p - 1u) & 31u));
         }
         wave_sync();
-        trans_windows<IT, false>(val + e, idx + e, T, nbk, 0u, k, y, ldy, direct, L, lane);
+        trans_windows<IT, false>(val + e, idx + e, T, nbk, 0u, k, y, ldy, scale, direct, L, lane);
         if (!direct) trans_flush(bcol, cb, nbk, k, y, ldy, L, lane);
         wave_sync();
         e += T;
@@ -1194,7 +1194,7 @@ __device__ __forceinline__ void trans_coo(MatPtr A_, uint32_t b0, uint32_t b1, u
 
 template <typename BT, typename RT>
 __device__ __forceinline__ void trans_csr(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, int64_t I, double *y,
-                                          int64_t ldy, TransLds &L, int lane)
+                                          int64_t ldy, double scale, TransLds &L, int lane)
 {
     if (b0 >= b1) return;
     const MatPtr A = opaque_s(A_);
@@ -1246,7 +1246,8 @@ __device__ __forceinline__ void trans_csr(MatPtr A_, uint32_t b0, uint32_t b1, u
                 }
             if (w) before = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan_dpp(before), kWave - 1);
             wave_sync();
-            trans_windows<uint8_t, true>(val + (e + w), ccol + (e + w), Tw, nseg, before, k, y, ldy, false, L, lane);
+            trans_windows<uint8_t, true>(val + (e + w), ccol + (e + w), Tw, nseg, before, k, y, ldy, scale, false, L,
+                                         lane);
             wave_sync();
         }
         trans_flush(bcol, cb, min(nb, b1 - cb), k, y, ldy, L, lane);
@@ -1257,7 +1258,7 @@ __device__ __forceinline__ void trans_csr(MatPtr A_, uint32_t b0, uint32_t b1, u
 // Bitmap or dense blocks, one at a time, lanes over the positions.
 template <typename BT, int SC>
 __device__ __forceinline__ void trans_bmdn(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, int64_t I, double *y,
-                                           int64_t ldy, TransLds &L, int lane)
+                                           int64_t ldy, double scale, TransLds &L, int lane)
 {
     if (b0 >= b1) return;
     const MatPtr A = opaque_s(A_);
@@ -1288,7 +1289,7 @@ __device__ __forceinline__ void trans_bmdn(MatPtr A_, uint32_t b0, uint32_t b1, 
             // zeros fill a dense block where it has no entry: not a product
             // (x there may be infinite)
             if (SC == DENSE) on = on && v != 0.0;
-            if (on && !(J == I && r == c)) atomicAdd(&L.acc[c], v * L.xs[r]);
+            if (on && !(J == I && r == c)) atomicAdd(&L.acc[c], (scale * v) * L.xs[r]);
         }
         trans_flush(bcol, b, 1u, k, y, ldy, L, lane);
     }
@@ -1309,6 +1310,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_spmv_trans(TransArgs)
     const double *x = glob<double>(P->x);
     double *y = glob_rw(P->y);
     const int64_t ldy = P->ldy;
+    const double scale = P->scale;
     int64_t I;
     uint32_t sc = 4, b0 = 0, b1 = 0, e0 = 0;  // scheme 4: a whole strip
     if (item < B->n_lstrips) {
@@ -1326,7 +1328,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_spmv_trans(TransArgs)
     for (int i = lane; i < kTransAcc; i += kWave) L.acc[i] = 0.0;
     for (int r = lane; r < s; r += kWave) {
         const int64_t gr = I * s + r;
-        L.xs[r] = gr < A->m ? P->scale * x[gr * P->ldx] : 0.0;
+        L.xs[r] = gr < A->m ? x[gr * P->ldx] : 0.0;
     }
     wave_sync();
     // (constant scheme arguments: see spmv_item)
@@ -1338,19 +1340,19 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_spmv_trans(TransArgs)
     uint32_t f, l, e;
     if (sc == 4 || sc == COO) {
         range(COO, f, l, e);
-        trans_coo<BT, IT>(A, f, l, e, I, y, ldy, P->direct != 0, L, lane);
+        trans_coo<BT, IT>(A, f, l, e, I, y, ldy, scale, P->direct != 0, L, lane);
     }
     if (sc == 4 || sc == CSR) {
         range(CSR, f, l, e);
-        trans_csr<BT, RT>(A, f, l, e, I, y, ldy, L, lane);
+        trans_csr<BT, RT>(A, f, l, e, I, y, ldy, scale, L, lane);
     }
     if (sc == 4 || sc == BITMAP) {
         range(BITMAP, f, l, e);
-        trans_bmdn<BT, BITMAP>(A, f, l, e, I, y, ldy, L, lane);
+        trans_bmdn<BT, BITMAP>(A, f, l, e, I, y, ldy, scale, L, lane);
     }
     if (sc == 4 || sc == DENSE) {
         range(DENSE, f, l, e);
-        trans_bmdn<BT, DENSE>(A, f, l, e, I, y, ldy, L, lane);
+        trans_bmdn<BT, DENSE>(A, f, l, e, I, y, ldy, scale, L, lane);
     }
 }
 

@@ -56,3 +56,23 @@ def test_dense_padding_times_a_non_finite_x(gpu, s, bad):
     ref = product(T, x)
     assert np.isfinite(ref[missing]).all() and not np.isfinite(ref[:s]).all()
     assert np.array_equal(got, ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("alpha,v,big", [(1e200, 1e-100, 1e150), (-1e-200, 1e200, 1e-150), (1e-200, 1e150, 1e200)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_products_that_stay_in_range_do(gpu, alpha, v, big, skew):
+    """(alpha v) x is taken as such, in all four schemes: alpha x alone would
+    be infinite, or zero."""
+    s = 32
+    rc = [block(s, I, 0, z, I) for I, z in ((1, 40), (2, 100), (3, 500), (4, 1020))]
+    r, c = np.concatenate([a for a, _ in rc]), np.concatenate([a for _, a in rc])
+    T = synth.from_triplets(5 * s, 5 * s, r, c, np.full(r.size, v))
+    x = np.full(T.n, big)
+    x[:s] = 1.0
+    print(f"case mirrored range alpha={alpha} v={v} x={big} skew={skew}", flush=True)
+    got, st = spmv(T, x, s, alpha, skew)
+    assert list(st["blocks"].values()) == [1, 1, 1, 1]
+    ref = product(T, x, alpha, skew)
+    assert np.isfinite(ref).all() and (ref[:s] != 0).all()
+    # sums of at most 1660 products of one sign: 2 * 1660 roundings at most
+    assert np.all(np.abs(got - ref) <= 2 * 1660 * 2.0 ** -53 * np.abs(ref))
