@@ -29,8 +29,15 @@ class DevBuf {
         release();
         n_ = bytes;
         if (bytes == 0) return;
-        hipError_t e = hipMalloc(&p_, bytes);
-        if (e != hipSuccess && scratch_trim()) e = hipMalloc(&p_, bytes);
+        // a failed call's error stays with the thread, past calls that succeed,
+        // until it is read: the next launch check would report it
+        auto get = [&] {
+            const hipError_t r = hipMalloc(&p_, bytes);
+            if (r != hipSuccess) (void)hipGetLastError();
+            return r;
+        };
+        hipError_t e = get();
+        if (e != hipSuccess && scratch_trim()) e = get();
         if (e != hipSuccess) {
             p_ = nullptr;
             n_ = 0;

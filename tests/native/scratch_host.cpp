@@ -1,0 +1,96 @@
+// The scratch of prims.hip on a stand-in for the HIP runtime: device memory is
+// a byte count with a limit, launches do nothing, and a failed call's error
+// stays with the thread until hipGetLastError reads it.
+//   scratch_host CASE     (exit status 0: the case holds)
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+
+#include "prims.hpp"
+
+namespace fake {
+size_t limit = (size_t)1 << 40, used = 0, most = 0;
+std::map<void *, size_t> live;
+thread_local hipError_t last = hipSuccess;
+uintptr_t next = 4096;
+}  // namespace fake
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n)
+{
+    if (fake::used + n > fake::limit) return fake::last = hipErrorOutOfMemory;
+    *p = (void *)fake::next;
+    fake::next += (n + 8191) & ~(size_t)4095;
+    fake::live[*p] = n;
+    fake::used += n;
+    if (fake::used > fake::most) fake::most = fake::used;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    if (!fake::live.count(p)) std::abort();
+    fake::used -= fake::live[p];
+    fake::live.erase(p);
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { hipError_t e = fake::last; fake::last = hipSuccess; return e; }
+const char *hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipMemcpyAsync(void *, const void *, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
+hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
+void **__hipRegisterFatBinary(const void *) { return nullptr; }
+void __hipRegisterFunction(void **, const void *, char *, const char *, unsigned, void *, void *, void *, void *, int *) {}
+void __hipUnregisterFatBinary(void **) {}
+}
+
+using namespace abhsf;
+
+#define CHECK(c)                                                     \
+    do {                                                             \
+        if (!(c)) {                                                  \
+            std::printf("line %d: %s does not hold\n", __LINE__, #c); \
+            return 1;                                                \
+        }                                                            \
+    } while (0)
+
+constexpr size_t MiB = (size_t)1 << 20;
+
+// One operation that used pieces of these sizes (MiB).
+static void operation(std::initializer_list<size_t> sizes)
+{
+    Arena a(nullptr);
+    for (size_t n : sizes) a.take_bytes(n * MiB);
+}
+
+// An allocation that succeeds after the kept scratch is freed leaves no error
+// behind for the next launch check; nor does one that fails for good.
+static int retry()
+{
+    operation({64, 32});
+    fake::limit = 120 * MiB;
+    DevBuf b(100 * MiB);
+    CHECK(b.get() != nullptr);
+    CHECK(hipGetLastError() == hipSuccess);
+    bool thrown = false;
+    try {
+        DevBuf c(100 * MiB);
+    } catch (const Error &e) {
+        thrown = e.code == ABHSF_ERR_ALLOC;
+    }
+    CHECK(thrown);
+    CHECK(hipGetLastError() == hipSuccess);
+    return 0;
+}
+
+int main(int argc, char **argv)
+{
+    const std::string c = argc > 1 ? argv[1] : "";
+    if (c == "retry") return retry();
+    return 2;
+}
