@@ -6,16 +6,23 @@
 #include "prims.hpp"
 
 #include <algorithm>
+#include <iterator>
 #include <mutex>
 #include <utility>
 
 namespace abhsf {
 namespace {
 
-// Scratch kept between operations, per device.
+// Scratch kept between operations.
+struct KeptBuf {
+    int device;
+    uint64_t at;  // when it was given back (Kept::now)
+    DevBuf buf;
+};
 struct Kept {
     std::mutex m;
-    std::vector<std::pair<int, DevBuf>> bufs;
+    uint64_t now = 0;
+    std::vector<KeptBuf> bufs;
 };
 Kept &kept()
 {
@@ -207,7 +214,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const uint64_t *__re
 
 bool scratch_trim()
 {
-    std::vector<std::pair<int, DevBuf>> out;
+    std::vector<KeptBuf> out;
     {
         std::lock_guard<std::mutex> l(kept().m);
         out.swap(kept().bufs);
@@ -219,16 +226,7 @@ Arena::Arena(hipStream_t st) : st_(st)
 {
     ABHSF_HIP(hipGetDevice(&device_));
     std::lock_guard<std::mutex> l(kept().m);
-    auto &b = kept().bufs;
-    for (size_t i = 0; i < b.size();) {
-        if (b[i].first != device_) {
-            i++;
-            continue;
-        }
-        kept_.push_back(std::move(b[i].second));
-        b[i] = std::move(b.back());
-        b.pop_back();
-    }
+    from_ = kept().now++;
 }
 
 Arena::~Arena()
@@ -236,15 +234,23 @@ Arena::~Arena()
     // nothing on the stream uses the buffers any more; after an error they go
     // back to the runtime
     if (hipStreamSynchronize(st_) != hipSuccess) return;
+    std::vector<KeptBuf> out;  // freed after the lock is given up
     try {
         std::lock_guard<std::mutex> l(kept().m);
+        auto &b = kept().bufs;
+        // what lay there all the while goes: this operation had no use for it
+        const auto stale = std::stable_partition(
+            b.begin(), b.end(), [&](const KeptBuf &q) { return q.device != device_ || q.at > from_; });
+        out.assign(std::make_move_iterator(stale), std::make_move_iterator(b.end()));
+        b.erase(stale, b.end());
         size_t total = 0;
-        for (const auto &b : kept().bufs)
-            if (b.first == device_) total += b.second.bytes();
-        for (auto &b : used_)
-            if (total + b.bytes() <= kScratchKeep) {
-                total += b.bytes();
-                kept().bufs.emplace_back(device_, std::move(b));
+        for (const auto &q : b)
+            if (q.device == device_) total += q.buf.bytes();
+        const uint64_t at = ++kept().now;
+        for (auto &q : used_)
+            if (total + q.bytes() <= kScratchKeep) {
+                total += q.bytes();
+                b.push_back({device_, at, std::move(q)});
             }
     } catch (...) {  // out of host memory: what is left is freed
     }
@@ -252,18 +258,22 @@ Arena::~Arena()
 
 void *Arena::fresh(size_t bytes)
 {
-    size_t best = kept_.size();
-    for (size_t i = 0; i < kept_.size(); i++)
-        if (kept_[i].bytes() >= bytes && kept_[i].bytes() <= 2 * bytes &&
-            (best == kept_.size() || kept_[i].bytes() < kept_[best].bytes()))
-            best = i;
-    if (best < kept_.size()) {
-        used_.push_back(std::move(kept_[best]));
-        kept_.erase(kept_.begin() + (std::ptrdiff_t)best);
-    } else {
-        DevBuf b(bytes);
-        used_.push_back(std::move(b));
+    used_.reserve(used_.size() + 1);
+    {
+        std::lock_guard<std::mutex> l(kept().m);
+        auto &b = kept().bufs;
+        size_t best = b.size();
+        for (size_t i = 0; i < b.size(); i++)
+            if (b[i].device == device_ && b[i].buf.bytes() >= bytes && b[i].buf.bytes() <= 2 * bytes &&
+                (best == b.size() || b[i].buf.bytes() < b[best].buf.bytes()))
+                best = i;
+        if (best < b.size()) {
+            used_.push_back(std::move(b[best].buf));
+            b.erase(b.begin() + (std::ptrdiff_t)best);
+            return used_.back().get();
+        }
     }
+    used_.emplace_back(bytes);
     return used_.back().get();
 }
 

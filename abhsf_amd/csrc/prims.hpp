@@ -68,9 +68,11 @@ class DevBuf {
 // at first, 28 ms once the clearing lags behind).  Small pieces share chunks;
 // the buffers of the last operation stay for the next one: at most
 // kScratchKeep bytes per device, no others than that operation used, and none
-// if an allocation fails.  An Arena owns what it took until it is destroyed,
-// after the stream has finished, so operations of several threads or streams
-// never share a buffer.  Pieces are 256-byte aligned.
+// if an allocation fails: an operation takes a kept buffer when it needs one of
+// its size, and the others stay where scratch_trim finds them.  An Arena owns
+// what it took until it is destroyed, after the stream has finished, so
+// operations of several threads or streams never share a buffer.  Pieces are
+// 256-byte aligned.
 constexpr size_t kScratchKeep = (size_t)1 << 30;
 
 class Arena {
@@ -86,7 +88,8 @@ class Arena {
   private:
     static constexpr size_t kChunk = (size_t)16 << 20;
     void *fresh(size_t bytes);  // a kept buffer that fits, or a new one
-    std::vector<DevBuf> kept_, used_;
+    std::vector<DevBuf> used_;
+    uint64_t from_ = 0;  // when the operation began (Kept::now)
     char *chunk_ = nullptr;
     size_t at_ = 0;
     int device_ = 0;

@@ -88,9 +88,33 @@ static int retry()
     return 0;
 }
 
+// Kept buffers that an open operation has not taken are freed when memory runs
+// out; one that it needs is taken, and one that it did not need is gone after.
+static int idle()
+{
+    operation({300, 200});
+    CHECK(fake::used == 500 * MiB);
+    {
+        Arena a(nullptr);
+        a.take_bytes(200 * MiB);
+        CHECK(fake::used == 500 * MiB);  // the kept one
+        fake::limit = 600 * MiB;
+        DevBuf b(350 * MiB);
+        CHECK(fake::used == 550 * MiB);
+    }
+    CHECK(fake::used == 200 * MiB);
+    operation({90, 50});
+    CHECK(fake::used == 140 * MiB);
+    fake::limit = (size_t)1 << 40;
+    operation({600, 600});  // above the bound: one of them
+    CHECK(fake::used == 600 * MiB);
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     const std::string c = argc > 1 ? argv[1] : "";
     if (c == "retry") return retry();
+    if (c == "idle") return idle();
     return 2;
 }
