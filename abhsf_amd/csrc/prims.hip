@@ -6,18 +6,20 @@
 #include "prims.hpp"
 
 #include <algorithm>
-#include <iterator>
 #include <mutex>
 #include <utility>
 
 namespace abhsf {
 namespace {
 
-// Scratch kept between operations.
+// Scratch kept between operations, or (owner) idle within one: its earlier use
+// may not have finished on the owner's stream.
 struct KeptBuf {
     int device;
     uint64_t at;  // when it was given back (Kept::now)
     DevBuf buf;
+    const Arena *owner = nullptr;
+    hipStream_t stream = nullptr;  // the owner's
 };
 struct Kept {
     std::mutex m;
@@ -217,6 +219,8 @@ bool scratch_trim()
     std::vector<KeptBuf> out;
     {
         std::lock_guard<std::mutex> l(kept().m);
+        for (const auto &q : kept().bufs)  // (under the lock: the owner cannot end meanwhile)
+            if (q.owner) (void)hipStreamSynchronize(q.stream);
         out.swap(kept().bufs);
     }
     return !out.empty();  // freed here
@@ -233,24 +237,36 @@ Arena::~Arena()
 {
     // nothing on the stream uses the buffers any more; after an error they go
     // back to the runtime
-    if (hipStreamSynchronize(st_) != hipSuccess) return;
-    std::vector<KeptBuf> out;  // freed after the lock is given up
+    const bool done = hipStreamSynchronize(st_) == hipSuccess;
+    std::lock_guard<std::mutex> l(kept().m);
+    auto &b = kept().bufs;
+    const uint64_t at = ++kept().now;
+    size_t total = 0;
+    for (const auto &q : b)
+        if (q.device == device_ && !q.owner && q.at > from_) total += q.buf.bytes();
+    for (size_t i = 0; i < b.size();) {
+        KeptBuf &q = b[i];
+        const bool mine = q.owner == this;
+        // what lay there all the while goes too: this operation had no use for it
+        const bool drop = mine ? !done || total + q.buf.bytes() > kScratchKeep
+                               : q.device == device_ && !q.owner && q.at <= from_;
+        if (drop) {
+            b.erase(b.begin() + (std::ptrdiff_t)i);
+            continue;
+        }
+        if (mine) {
+            q.owner = nullptr;
+            q.at = at;
+            total += q.buf.bytes();
+        }
+        i++;
+    }
+    if (!done) return;
     try {
-        std::lock_guard<std::mutex> l(kept().m);
-        auto &b = kept().bufs;
-        // what lay there all the while goes: this operation had no use for it
-        const auto stale = std::stable_partition(
-            b.begin(), b.end(), [&](const KeptBuf &q) { return q.device != device_ || q.at > from_; });
-        out.assign(std::make_move_iterator(stale), std::make_move_iterator(b.end()));
-        b.erase(stale, b.end());
-        size_t total = 0;
-        for (const auto &q : b)
-            if (q.device == device_) total += q.buf.bytes();
-        const uint64_t at = ++kept().now;
         for (auto &q : used_)
             if (total + q.bytes() <= kScratchKeep) {
-                total += q.bytes();
                 b.push_back({device_, at, std::move(q)});
+                total += b.back().buf.bytes();
             }
     } catch (...) {  // out of host memory: what is left is freed
     }
@@ -264,8 +280,8 @@ void *Arena::fresh(size_t bytes)
         auto &b = kept().bufs;
         size_t best = b.size();
         for (size_t i = 0; i < b.size(); i++)
-            if (b[i].device == device_ && b[i].buf.bytes() >= bytes && b[i].buf.bytes() <= 2 * bytes &&
-                (best == b.size() || b[i].buf.bytes() < b[best].buf.bytes()))
+            if (b[i].device == device_ && (!b[i].owner || b[i].owner == this) && b[i].buf.bytes() >= bytes &&
+                b[i].buf.bytes() <= 2 * bytes && (best == b.size() || b[i].buf.bytes() < b[best].buf.bytes()))
                 best = i;
         if (best < b.size()) {
             used_.push_back(std::move(b[best].buf));
@@ -275,6 +291,19 @@ void *Arena::fresh(size_t bytes)
     }
     used_.emplace_back(bytes);
     return used_.back().get();
+}
+
+void Arena::to_idle(size_t first)
+{
+    try {
+        std::lock_guard<std::mutex> l(kept().m);
+        auto &b = kept().bufs;
+        b.reserve(b.size() + used_.size() - first);
+        for (size_t i = first; i < used_.size(); i++)
+            b.push_back({device_, kept().now, std::move(used_[i]), this, st_});
+        used_.resize(first);
+    } catch (...) {  // out of host memory: they stay in use to the end
+    }
 }
 
 void *Arena::take_bytes(size_t bytes)
@@ -307,6 +336,7 @@ void radix_sort_pairs(uint64_t *keys, uint32_t *vals, uint64_t n, int key_bits, 
     ABHSF_REQUIRE(n < (1ull << 32), ABHSF_ERR_UNSUPPORTED, "radix sort limited to 2^32 elements");
     const uint64_t ntiles = (n + kTile - 1) / kTile;
     ABHSF_REQUIRE(ntiles * kRadix < (1ull << 32), ABHSF_ERR_UNSUPPORTED, "radix histogram too large");
+    const Arena::Scope scope(tmp);
     uint64_t *ka = keys, *kb = tmp.take<uint64_t>(n);
     uint32_t *va = vals, *vb = tmp.take<uint32_t>(n);
     uint32_t *hist = tmp.take<uint32_t>(ntiles * kRadix);

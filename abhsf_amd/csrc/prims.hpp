@@ -85,9 +85,32 @@ class Arena {
     template <typename T>
     T *take(uint64_t n) { return static_cast<T *>(take_bytes((size_t)n * sizeof(T))); }
 
+    // Pieces taken in a scope are idle after it: later pieces of the Arena
+    // (on the same stream, so in order) take their place, and they are freed
+    // if an allocation fails.
+    class Scope {
+      public:
+        explicit Scope(Arena &a) : a_(a), first_(a.used_.size()), chunk_(a.chunk_), at_(a.at_) {}
+        ~Scope()
+        {
+            a_.chunk_ = chunk_;
+            a_.at_ = at_;
+            a_.to_idle(first_);
+        }
+        Scope(const Scope &) = delete;
+        Scope &operator=(const Scope &) = delete;
+
+      private:
+        Arena &a_;
+        size_t first_;
+        char *chunk_;
+        size_t at_;
+    };
+
   private:
     static constexpr size_t kChunk = (size_t)16 << 20;
     void *fresh(size_t bytes);  // a kept buffer that fits, or a new one
+    void to_idle(size_t first);  // used_[first ..]
     std::vector<DevBuf> used_;
     uint64_t from_ = 0;  // when the operation began (Kept::now)
     char *chunk_ = nullptr;

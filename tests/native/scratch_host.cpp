@@ -111,10 +111,31 @@ static int idle()
     return 0;
 }
 
+// What the sort took is not held for the rest of its operation: later pieces
+// take its place, and an allocation that needs the memory gets it.
+static int sorted()
+{
+    constexpr uint64_t n = (uint64_t)16 << 20;
+    Arena a(nullptr);
+    uint64_t *keys = a.take<uint64_t>(n);
+    uint32_t *vals = a.take<uint32_t>(n);
+    const size_t before = fake::used;
+    radix_sort_pairs(keys, vals, n, 24, nullptr, a);
+    const size_t after = fake::used;
+    CHECK(after >= before + 12 * n);
+    a.take<uint64_t>(n);
+    CHECK(fake::used == after);
+    fake::limit = after;
+    DevBuf b(4 * n);  // the sort's second values
+    CHECK(fake::used <= after);
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     const std::string c = argc > 1 ? argv[1] : "";
     if (c == "retry") return retry();
     if (c == "idle") return idle();
+    if (c == "sorted") return sorted();
     return 2;
 }
