@@ -275,13 +275,16 @@ Arena::~Arena()
 void *Arena::fresh(size_t bytes)
 {
     used_.reserve(used_.size() + 1);
+    // a kept buffer of at most 1/8 more: the builds of one matrix size ask for
+    // the same sizes, and more would be memory that nothing can give back
+    const size_t most = bytes + bytes / 8;
     {
         std::lock_guard<std::mutex> l(kept().m);
         auto &b = kept().bufs;
         size_t best = b.size();
         for (size_t i = 0; i < b.size(); i++)
             if (b[i].device == device_ && (!b[i].owner || b[i].owner == this) && b[i].buf.bytes() >= bytes &&
-                b[i].buf.bytes() <= 2 * bytes && (best == b.size() || b[i].buf.bytes() < b[best].buf.bytes()))
+                b[i].buf.bytes() <= most && (best == b.size() || b[i].buf.bytes() < b[best].buf.bytes()))
                 best = i;
         if (best < b.size()) {
             used_.push_back(std::move(b[best].buf));

@@ -131,11 +131,24 @@ static int sorted()
     return 0;
 }
 
+// A piece does not hold a kept buffer much larger than itself.
+static int fitting()
+{
+    operation({200});
+    fake::limit = 250 * MiB;
+    Arena a(nullptr);
+    a.take_bytes(100 * MiB);
+    DevBuf b(120 * MiB);
+    CHECK(fake::used == 220 * MiB);
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     const std::string c = argc > 1 ? argv[1] : "";
     if (c == "retry") return retry();
     if (c == "idle") return idle();
     if (c == "sorted") return sorted();
+    if (c == "fitting") return fitting();
     return 2;
 }

@@ -27,7 +27,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["retry", "idle", "sorted"])
+@pytest.mark.parametrize("case", ["retry", "idle", "sorted", "fitting"])
 def test_scratch(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
