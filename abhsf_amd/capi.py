@@ -31,7 +31,7 @@ EXPORTED = (
     "abhsf_batch_spmv", "abhsf_batch_synchronize", "abhsf_batch_profile", "abhsf_batch_destroy", "abhsf_synchronize",
     "abhsf_destroy", "abhsf_last_error", "abhsf_version", "abhsf_set_symmetry",
     "abhsf_delta_create", "abhsf_delta_create_codec", "abhsf_delta_build_csr", "abhsf_delta_spmv", "abhsf_delta_get_stats",
-    "abhsf_delta_export", "abhsf_delta_synchronize", "abhsf_delta_destroy",
+    "abhsf_delta_export", "abhsf_delta_synchronize", "abhsf_delta_destroy", "abhsf_scratch_trim",
 )
 
 
@@ -138,6 +138,7 @@ def lib():
         L.abhsf_batch_destroy.argtypes = [vp]
         L.abhsf_synchronize.argtypes = [vp]
         L.abhsf_destroy.argtypes = [vp]
+        L.abhsf_scratch_trim.argtypes = [C.POINTER(C.c_uint64)]
         L.abhsf_last_error.restype = C.c_char_p
         L.abhsf_last_error.argtypes = []
         L.abhsf_version.restype = C.c_char_p
@@ -147,6 +148,7 @@ def lib():
                 getattr(L, name).restype = C.c_int32
         L.abhsf_mlp_num_params.restype = C.c_int64
         _lib = L
+        hip.reclaim = scratch_trim
     return _lib
 
 
@@ -155,3 +157,10 @@ def call(fn: str, *args) -> None:
     rc = getattr(L, fn)(*args)
     if rc != OK:
         raise AbhsfError(fn, rc, L.abhsf_last_error().decode())
+
+
+def scratch_trim() -> int:
+    """Frees the device scratch kept between conversions; the bytes freed."""
+    n = C.c_uint64(0)
+    call("abhsf_scratch_trim", C.byref(n))
+    return n.value

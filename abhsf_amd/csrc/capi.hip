@@ -409,6 +409,14 @@ abhsf_status abhsf_export(const abhsf_handle *h, const char *name, void *dst, si
     });
 }
 
+abhsf_status abhsf_scratch_trim(uint64_t *freed)
+{
+    return guarded([&] {
+        const size_t n = abhsf::scratch_trim();
+        if (freed) *freed = n;
+    });
+}
+
 abhsf_status abhsf_block_hist(const int64_t *rowptr, const int32_t *col, int64_t m, int64_t n, int64_t nnz,
                               int32_t on_device, int32_t kr, int32_t ks, int64_t strip_stride, uint64_t *hist,
                               int64_t hist_cap, uint64_t *nblocks, uint64_t *sampled_nnz, void *stream)

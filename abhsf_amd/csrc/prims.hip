@@ -214,7 +214,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const uint64_t *__re
 
 }  // namespace
 
-bool scratch_trim()
+size_t scratch_trim()
 {
     std::vector<KeptBuf> out;
     {
@@ -223,7 +223,9 @@ bool scratch_trim()
             if (q.owner) (void)hipStreamSynchronize(q.stream);
         out.swap(kept().bufs);
     }
-    return !out.empty();  // freed here
+    size_t bytes = 0;
+    for (const auto &q : out) bytes += q.buf.bytes();
+    return bytes;  // freed here
 }
 
 Arena::Arena(hipStream_t st) : st_(st)

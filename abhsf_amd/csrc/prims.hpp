@@ -7,8 +7,8 @@
 
 namespace abhsf {
 
-// Frees the scratch kept between operations (Arena); false if there was none.
-bool scratch_trim();
+// Frees the scratch kept between operations (Arena); its bytes.
+size_t scratch_trim();
 
 // RAII device buffer.
 class DevBuf {

@@ -13,6 +13,7 @@ import numpy as np
 
 _ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 _hip = None
+reclaim = None  # frees device memory that can be spared, returns its bytes (set by capi.lib())
 
 H2D, D2H, D2D = 1, 2, 3
 
@@ -93,7 +94,12 @@ class DeviceArray:
         self.nbytes = int(np.prod(self.shape, dtype=np.int64)) * self.dtype.itemsize
         self.ptr = C.c_void_p(0)
         if self.nbytes:
-            check(_load().hipMalloc(C.byref(self.ptr), self.nbytes), f"hipMalloc({self.nbytes})")
+            rc = _load().hipMalloc(C.byref(self.ptr), self.nbytes)
+            if rc != 0:
+                _load().hipGetLastError()  # (it would stay with the thread)
+                if reclaim is not None and reclaim():
+                    rc = _load().hipMalloc(C.byref(self.ptr), self.nbytes)
+            check(rc, f"hipMalloc({self.nbytes})")
 
     @classmethod
     def from_numpy(cls, a: np.ndarray) -> "DeviceArray":

@@ -105,6 +105,13 @@ class abhsf_matrix {
         check(abhsf_spmm(h_, nrhs, alpha, X, ldx, beta, Y, ldy), "abhsf_spmm");
     }
 
+    // Frees the device scratch kept between conversions; its bytes.
+    static uint64_t scratch_trim()
+    {
+        uint64_t n = 0;
+        check(abhsf_scratch_trim(&n), "abhsf_scratch_trim");
+        return n;
+    }
     void synchronize() { check(abhsf_synchronize(h_), "abhsf_synchronize"); }
 
     abhsf_stats stats() const

@@ -187,6 +187,12 @@ abhsf_status abhsf_export(const abhsf_handle *h, const char *name, void *dst, si
 abhsf_status abhsf_import(abhsf_handle *h, int64_t m, int64_t n, int64_t nnz, int32_t count,
                           const char *const *names, const void *const *data, const size_t *bytes);
 
+/* Conversions and block statistics keep the device scratch of the last one for
+ * the next (at most 1 GiB per device).  It is freed when an allocation of this
+ * library runs out of memory, and by this call; *freed (may be NULL) receives
+ * the bytes.  May be called at any time, from any thread. */
+abhsf_status abhsf_scratch_trim(uint64_t *freed);
+
 /* Block statistics on the GPU: hist[z] = number of nonzero r x s blocks
  * (r = 2^kr, s = 2^ks, 0 <= kr, ks <= 16) holding z entries (z >= hist_cap - 1
  * lands in hist[hist_cap - 1]); *nblocks = number of nonzero blocks.  Only

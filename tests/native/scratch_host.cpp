@@ -143,6 +143,24 @@ static int fitting()
     return 0;
 }
 
+// The call that gives the memory back says how much it was; an operation that
+// runs goes on.
+static int trim()
+{
+    operation({64, 32});
+    Arena a(nullptr);
+    void *p = a.take_bytes(32 * MiB);
+    CHECK(scratch_trim() == 64 * MiB);
+    CHECK(fake::used == 32 * MiB && fake::live.count(p));
+    {
+        const Arena::Scope scope(a);
+        a.take_bytes(40 * MiB);
+    }
+    CHECK(scratch_trim() == 40 * MiB);
+    CHECK(scratch_trim() == 0);
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     const std::string c = argc > 1 ? argv[1] : "";
@@ -150,5 +168,6 @@ int main(int argc, char **argv)
     if (c == "idle") return idle();
     if (c == "sorted") return sorted();
     if (c == "fitting") return fitting();
+    if (c == "trim") return trim();
     return 2;
 }

@@ -27,7 +27,45 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["retry", "idle", "sorted", "fitting"])
+@pytest.mark.parametrize("case", ["retry", "idle", "sorted", "fitting", "trim"])
 def test_scratch(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_device_array_reclaims(monkeypatch):
+    """A DeviceArray that runs out of memory has the kept scratch freed first."""
+    from abhsf_amd import hip
+
+    class Runtime:
+        free, error = 100, 0
+
+        def hipMalloc(self, p, n):
+            if n > self.free:
+                self.error = 2
+                return 2
+            self.free -= n
+            return 0
+
+        def hipGetLastError(self):
+            self.error = 0
+
+        def hipFree(self, p):
+            return 0
+
+        def hipGetErrorString(self, rc):
+            return b"out of memory"
+
+    rt, calls = Runtime(), []
+
+    def reclaim():
+        calls.append(1)
+        rt.free += 300
+        return 300
+
+    monkeypatch.setattr(hip, "_hip", rt)
+    monkeypatch.setattr(hip, "reclaim", reclaim)
+    hip.DeviceArray(40)
+    assert calls == [1] and rt.error == 0
+    with pytest.raises(hip.HipError):
+        hip.DeviceArray(1000)
