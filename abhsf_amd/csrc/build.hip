@@ -501,7 +501,6 @@ SpmvLaunch Storage::launch() const
     SpmvLaunch L;
     L.bcol_bytes = bcol_bytes;
     L.val_bytes = val_bytes;
-    L.coo_direct = ne[COO] < 2 * nb[COO];
     L.has_dense = nb[DENSE] > 0;
     L.bal.light = bal_light.get<uint32_t>();
     L.bal.pack = bal_pack.get<uint32_t>();

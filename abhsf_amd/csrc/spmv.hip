@@ -1055,9 +1055,10 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_spmv_strip(StripArgs)
 // ===========================================================================
 
 // A wave takes one strip (or unit).  Its x rows are kept in LDS, and the
-// products (scale v) x (scale x may leave the range where scale v does not) of up to kTransAcc / s blocks are summed by column in LDS before
-// they are added to y, 64 consecutive columns per wave instruction; COO blocks
-// of fewer than two entries on average (direct) are added entry by entry.
+// products (scale v) x (scale x may leave the range where scale v does not) of
+// up to kTransAcc / s blocks are summed by column in LDS before they are added
+// to y, 64 consecutive columns per wave instruction.  Scattered COO blocks are
+// added entry by entry, 256 blocks at a time (trans_coo).
 // Bound: the global adds, which the fabric takes one request at a time.  With
 // an add for every entry (about 31 requests per wave instruction) the 27-point
 // stencil 99^3, s = 64, one triangle took 262 us for this pass, now about 70.
@@ -1070,7 +1071,6 @@ struct TransArgs {
     double *y;
     int64_t ldx, ldy;
     double scale;
-    int direct;
 };
 
 struct TransLds {
@@ -1136,9 +1136,21 @@ __device__ __forceinline__ void trans_windows(const double *__restrict__ vp, con
     }
 }
 
+// COO blocks.  The sums by column pay where the chunk of kTransAcc / s blocks
+// holds entries for half of its columns or more; below, the chunk is a handful
+// of entries between two passes over the sums, and the entries are added to y
+// as they come, in chunks of up to 256 blocks that end at the next block that
+// holds entries for half of its columns.  With the sums everywhere (a mean of two entries a block over
+// the matrix) one triangle of 2e5 uniform random columns, 8 a row, took 1255
+// us at s = 256 (55 now), 32 a row at s = 128 1770 us (174), R-MAT scale 16 at
+// s = 256 370 us (76).  The line at s / 4: uniform n = 2e4, 32 a row, s = 256
+// 135 us (50 here); at 3 s / 4: stencil 99^3 s = 256 96 us (74 here).  Up to
+// s = 8 a block's columns lie in one line, and the line is at 3 s / 4: R-MAT
+// scale 16 s = 8 240 us at s / 2, 235 here; never: an arrow of n = 1e5, whose
+// strips all add to column 0, 1211 us, 161 here.
 template <typename BT, typename IT>
 __device__ __forceinline__ void trans_coo(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, int64_t I, double *y,
-                                          int64_t ldy, double scale, bool direct, TransLds &L, int lane)
+                                          int64_t ldy, double scale, TransLds &L, int lane)
 {
     if (b0 >= b1) return;
     const MatPtr A = opaque_s(A_);
@@ -1148,20 +1160,47 @@ __device__ __forceinline__ void trans_coo(MatPtr A_, uint32_t b0, uint32_t b1, u
     const uint16_t *__restrict__ z1 = glob<uint16_t>(A->z1[COO]);
     const BT *__restrict__ bcol = glob<BT>(A->bcol[COO]);
     uint32_t *ends32 = reinterpret_cast<uint32_t *>(L.w.ends);
-    const uint32_t cap = direct ? (uint32_t)kSegs : min((uint32_t)kTransAcc >> k, (uint32_t)kSegs);
-    uint32_t cb = b0;
+    const uint32_t cap = min((uint32_t)kTransAcc >> k, (uint32_t)kSegs);
+    const uint32_t full = k > 3 ? 1u << (k - 1) : max(2u, (3u << k) >> 2);
+    uint32_t cb = b0, look = (uint32_t)kSegs;  // blocks to look at
 #pragma unroll 1
     while (cb < b1) {
-        uint32_t nbk = min(cap, b1 - cb), z[4], bc[4], zs = 0;
+        uint32_t nbk = min(look, b1 - cb), z[4], bc[4], zs = 0;
         load4(z1, cb, nbk, lane, z);
         load4(bcol, cb, nbk, lane, bc);
+        // the first `cap` blocks' entries, and the first such block after them
+        uint32_t f = 4;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            z[i] = 4u * (uint32_t)lane + (uint32_t)i < nbk ? z[i] + 1u : 0u;
+        for (int i = 3; i >= 0; i--) {
+            const uint32_t j = 4u * (uint32_t)lane + (uint32_t)i;
+            z[i] = j < nbk ? z[i] + 1u : 0u;
             zs += z[i];
+            if (j >= cap && z[i] >= full) f = (uint32_t)i;
         }
-        const uint32_t incl = wave_incl_scan_dpp(zs);
-        uint32_t T = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        uint32_t incl = wave_incl_scan_dpp(zs);
+        const uint32_t first = cap < 4u ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(z[0] + z[1]))
+                                        : (uint32_t)__builtin_amdgcn_readlane((int)incl, (int)(cap / 4u) - 1);
+        const uint32_t ncap = min(cap, nbk);
+        const bool direct = first < ncap * full;  // uniform; (so a chunk always holds a block)
+        if (direct) {
+            const uint64_t any = __ballot(f < 4u);
+            if (any) {
+                const int l = __builtin_ctzll(any);
+                nbk = 4u * (uint32_t)l + (uint32_t)__builtin_amdgcn_readlane((int)f, l);
+            }
+        } else {
+            nbk = ncap;
+        }
+        look = direct ? (uint32_t)kSegs : cap;
+        // without the blocks from nbk on (the sums of later lanes are not used)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (4u * (uint32_t)lane + (uint32_t)i >= nbk) {
+                incl -= z[i];
+                zs -= z[i];
+                z[i] = 0u;
+            }
+        uint32_t T = (uint32_t)__builtin_amdgcn_readlane((int)incl, (int)((nbk - 1u) >> 2));
         bool mine = true;
         if (T > (uint32_t)kMaskEnts) {  // uniform: take the lanes whose blocks fit
             mine = incl <= (uint32_t)kMaskEnts;
@@ -1340,7 +1379,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void k_spmv_trans(TransArgs)
     uint32_t f, l, e;
     if (sc == 4 || sc == COO) {
         range(COO, f, l, e);
-        trans_coo<BT, IT>(A, f, l, e, I, y, ldy, scale, P->direct != 0, L, lane);
+        trans_coo<BT, IT>(A, f, l, e, I, y, ldy, scale, L, lane);
     }
     if (sc == 4 || sc == CSR) {
         range(CSR, f, l, e);
@@ -2167,7 +2206,7 @@ void spmv_transposed(const SpmvLaunch &L, const DevMat &A, int nrhs, double scal
     ABHSF_REQUIRE(nblk < (1ll << 31), ABHSF_ERR_UNSUPPORTED, "too many strips");
     const bool b16 = L.bcol_bytes == 2;
     for (int j = 0; j < nrhs; j++) {
-        const TransArgs args{A, b, X + j, Y + j, ldx, ldy, scale, L.coo_direct ? 1 : 0};
+        const TransArgs args{A, b, X + j, Y + j, ldx, ldy, scale};
 #define ABHSF_TRANS(BT_, IT_, RT_) \
     hipLaunchKernelGGL((k_spmv_trans<BT_, IT_, RT_>), dim3((unsigned)nblk), dim3(64 * kStripWaves), 0, st, args)
         if (A.s <= 8) {

@@ -79,7 +79,6 @@ constexpr uint32_t kNoItem = 0xFFFFFFFFu;
 struct SpmvLaunch {
     int bcol_bytes;          // 2 or 4
     int val_bytes;           // 8 (f64) or 4 (f32, compensated accumulation)
-    bool coo_direct = false; // COO blocks hold fewer than two entries on average
     bool has_dense = false;  // some dense-scheme blocks (SpMM: matrix-core tiles at R >= 16)
     Balance bal;
 };
