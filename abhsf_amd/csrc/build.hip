@@ -516,7 +516,7 @@ SpmvLaunch Storage::launch() const
     L.bal.n_slots = n_slots;
     L.bal.n_fix = n_fix;
     L.bal.tiled = tiled;
-    L.bal.tile_sweep = tile_sweep;
+    L.bal.tile_windows = tile_windows;
     L.bal.coo_rng = bal_coo_rng.get<uint32_t>();
     return L;
 }
@@ -582,7 +582,8 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
     bal_order.release();
     bal_coo_rng.release();
     n_light = n_units = n_heavy = n_slots = n_fix = 0;
-    tile_zs1 = tile_sweep = false;
+    tile_zs1 = false;
+    tile_windows = 4;
     if (unit <= 0 || M == 0) return;
     ABHSF_REQUIRE(panels == 1 || panels == kXcdCount, ABHSF_ERR_INVALID, "column panels must match the XCD count");
     ABHSF_REQUIRE(tile_rows <= 0 || panels == 1, ABHSF_ERR_INVALID, "tiles and column panels do not combine");
@@ -826,8 +827,8 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
         }
         // Blocks of 3 or more entries among the tiles' COO blocks (z - 1 >= 2):
         // below one in 64 the tiles are scattered, every gather a line of its
-        // own (uniform scatter: none; R-MAT scale 22: 9 %), and from n = 2^21
-        // on (x = 16 MB, four L2s) their sweep has to be kept together.
+        // own (uniform scatter: none; R-MAT scale 22: 9 %), and over a large x
+        // their sweep has to be kept together (Balance::tile_windows).
         uint64_t tile_blocks = 0, tile_ge3 = 0;
         for (size_t q = 0; q < items.size(); q++) {
             if (!tile[q] || items[q].size() < 2) continue;
@@ -837,7 +838,7 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
             }
         }
         tile_zs1 = tile_blocks > 0 && 64 * tile_ge3 >= tile_blocks;
-        tile_sweep = tile_blocks > 0 && !tile_zs1 && n > kSweepCols;
+        if (tile_blocks > 0 && !tile_zs1) tile_windows = n > kOneWindowCols ? 1 : n > kTwoWindowCols ? 2 : 4;
         // tiles first: they start together and sweep x in step (their COO
         // streams run in block-column order), the other items fill the
         // remaining slots and follow

@@ -509,7 +509,7 @@ enum CooMode { COO_STRIP, COO_TILE, COO_GROUP };
 
 template <typename VT, typename BT, typename IT, bool COMP, int MODE = COO_STRIP>
 __device__ __forceinline__ void coo_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
-                                       const Acc &acc, WaveLds &L, int lane_, bool sweep = false, int64_t I0 = 0,
+                                       const Acc &acc, WaveLds &L, int lane_, int windows = 4, int64_t I0 = 0,
                                        int T_ = 1)
 {
     if (b0 >= b1) return;
@@ -564,10 +564,12 @@ __device__ __forceinline__ void coo_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
             if (z[i] && mine) atomicOr(&ends32[(p - 1u) >> 5], 1u << ((p - 1u) & 31u));
         }
         wave_sync();
-        // one window in flight keeps the tiles' common sweep of a large x
-        // together (Balance::tile_sweep)
-        if (TILE && sweep)
+        // few windows in flight keep the tiles' common sweep of a large x
+        // together (Balance::tile_windows)
+        if (TILE && windows == 1)
             seg_windows<VT, IT, COMP, SEG_STRIPS, 1>(val + e, idx + e, T, nbk, 0u, k, x, acc, L, lane);
+        else if (TILE && windows == 2)
+            seg_windows<VT, IT, COMP, SEG_STRIPS, 2>(val + e, idx + e, T, nbk, 0u, k, x, acc, L, lane);
         else
             seg_windows<VT, IT, COMP, MODE == COO_STRIP ? SEG_COO : SEG_STRIPS, 4>(val + e, idx + e, T, nbk, 0u, k, x,
                                                                                    acc, L, lane);
@@ -940,8 +942,8 @@ __device__ __forceinline__ void spmv_item(MatPtr A, BalPtr B, int64_t item, cons
             // consecutive strips; rows (position << k) + lrow
             const int rows = T * s;
             clear(rows);
-            if (tiled) coo_r1<VT, BT, IT, COMP, COO_TILE>(A, tb0, tb1, te0, x, acc, L, lane, B->tile_sweep);
-            else coo_r1<VT, BT, IT, COMP, COO_GROUP>(A, tb0, tb1, te0, x, acc, L, lane, false, I, T);
+            if (tiled) coo_r1<VT, BT, IT, COMP, COO_TILE>(A, tb0, tb1, te0, x, acc, L, lane, B->tile_windows);
+            else coo_r1<VT, BT, IT, COMP, COO_GROUP>(A, tb0, tb1, te0, x, acc, L, lane, 4, I, T);
             csr_r1<VT, BT, RT, COMP>(A, r0, r1, re, x, acc, L, lane, I, T);
             if constexpr (sizeof(IT) == 1) {  // s <= 16
                 wave_sync();

@@ -32,14 +32,21 @@ struct Balance {
     // b1, first value, 0 for a tile}, in (block column, strip) order.
     bool tiled = false;
     const uint32_t *coo_rng = nullptr;  // [n_light][4]
-    // Scattered tiles over a large x (build_balance): their waves take one
-    // window of 64 entries at a time, four otherwise.  Tiles sweep x in block
-    // column order together; with more gathers in flight the fabric is busy
-    // enough that some waves fall behind, and x (beyond the L2s) is then read
-    // again for them.  block_mix s = 32, one / four windows: n = 2^22 430 /
-    // 550 us (L2 misses 27 M with four), 2.5 M 249 / 265, 2 M 202 / 198,
-    // 1 M 134 / 102 us.
-    bool tile_sweep = false;
+    // Windows of 64 entries that a tile's wave has in flight: four, and over a
+    // large x, where the tiles are scattered (build_balance), two or one.
+    // Tiles sweep x in block column order together; with more gathers in flight
+    // the fabric is busy enough that some waves fall behind, and x (beyond the
+    // L2s) is then read again for them (block_mix n = 2^22: 27 M L2 misses with
+    // four, 15 M with one).  s = 32, us with four / two / one windows:
+    //   n           uniform, 8 a row   uniform, 24 a row   block_mix
+    //   1.0 M        55 /  57 /  67     201 /  194 /  208   102 / 112 / 134
+    //   1.5 M        82 /  75 /  80     331 /  317 /  290   148 / 156 / 169
+    //     (FP32     109 /  96 /  96     298 /  294 /  336   128 / 127 / 127)
+    //   2.0 M       158 / 112 / 111     483 /  465 /  475   199 / 200 / 208
+    //     (FP32     172 / 146 / 115     418 /  373 /  409   194 / 185 / 181)
+    //   2.5 M       261 / 235 / 176     736 /  680 /  590   270 / 257 / 255
+    //   4.0 M       499 / 473 / 366    1511 / 1476 / 1144   548 / 515 / 428 (2^22)
+    int tile_windows = 4;
 };
 
 #ifndef ABHSF_TILE_WORK
@@ -64,7 +71,8 @@ constexpr int64_t kTileWork = ABHSF_TILE_WORK;  // entries per tile at most
 constexpr int kGroupRows = 256;
 constexpr int64_t kGroupWork = 2048;
 constexpr int64_t kGroupItems = 2048;
-constexpr int64_t kSweepCols = 1 << 21;         // columns above which scattered tiles sweep x in step
+constexpr int64_t kTwoWindowCols = 5 << 18;     // columns above which scattered tiles have two windows in flight
+constexpr int64_t kOneWindowCols = 7 << 18;     // and one
 
 constexpr int kXcdCount = 8;            // XCDs of an MI355X; workgroups go round-robin
 // Waves per workgroup of the single-RHS strip kernel.  Each wave runs its own

@@ -28,7 +28,7 @@ struct Storage {
     // its low coo_zb bits and the strip within the tile above them
     bool tiled = false;
     bool tile_zs1 = false;    // one in 64 or more of the tiles' COO blocks holds 3 or more entries
-    bool tile_sweep = false;  // scattered tiles over a large x (see Balance)
+    int tile_windows = 4;     // in flight per tile (see Balance)
     int coo_zb = 16;
     DevBuf bal_coo_rng;  // tiled: [n_light][4] of each item (Balance::coo_rng)
     // entries of the largest strip (dense blocks: positions), for the SpMM
