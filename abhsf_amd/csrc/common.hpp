@@ -107,6 +107,7 @@ __device__ inline double group_sum(double v)
 enum : int {
     DPP_QUAD_XOR1 = 0xB1,   // quad_perm [1,0,3,2]
     DPP_QUAD_XOR2 = 0x4E,   // quad_perm [2,3,0,1]
+    DPP_ROW_SHL1 = 0x101,   // lane i <- i + 1 within a row
     DPP_ROW_SHR1 = 0x111,
     DPP_ROW_SHR2 = 0x112,
     DPP_ROW_SHR4 = 0x114,

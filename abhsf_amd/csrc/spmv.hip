@@ -218,7 +218,7 @@ __device__ __forceinline__ void load4(const T *__restrict__ a, uint32_t cb, uint
 }
 
 // How an entry's row and column follow from its index and its segment.
-enum SegMode { SEG_COO, SEG_STRIPS, SEG_CSR };  // (one strip, several, CSR rows)
+enum SegMode { SEG_COO, SEG_STRIPS, SEG_CSR };  // (one strip, several, CSR rows with FP32 values)
 
 // Windows of 64 consecutive entries from vp / ip on (values and in-block
 // indices: COO (lrow << k) | lcol, CSR lcol), T <= kMaskEnts entries in nseg
@@ -297,7 +297,7 @@ __device__ __forceinline__ void seg_windows(const VT *__restrict__ vp, const IT 
     // 32-row random blocks s = 128 41 -> 25 us.  COO blocks of few entries
     // have no such runs (R-MAT scale 20 s = 256, 6 a block: 66 us, 71 this
     // way) except where the adds return (FP32 values).
-    if (U == 4 && (COMP || MODE == SEG_CSR || T >= 16u * nseg)) {
+    if (U == 4 && (COMP || T >= 16u * nseg)) {
 #pragma unroll 1
         for (; q + (uint32_t)(4 * kWave) <= T; q += (uint32_t)(4 * kWave)) {
             VT vw[4];
@@ -368,11 +368,96 @@ __device__ __forceinline__ void seg_windows(const VT *__restrict__ vp, const IT 
     else if (left) windows(q, integral_constant<int, 1>{}, std::true_type{});
 }
 
+// CSR entries of a mask (FP64 values; vp, ip, T, nseg, before as in
+// seg_windows): four consecutive entries per lane, a row (segment) summed by
+// fma from entry to entry.  A lane's open sum takes in the next lane's first
+// one if the row ends there (not across 16 lanes), so most rows of up to eight
+// entries are added once to the strip's sums.
+// Every entry added by itself (seg_windows) took 1 to 6 % less time (27-point
+// stencil 160^3 s = 64 250 us, here 253; s = 128 250, here 265), but rounded
+// each product and let a row's small terms meet the strip's sum one by one:
+// 32 % more error (rms) for the stencil at s = 32, 25 % at s = 64.
+__device__ __forceinline__ void csr_sums(const double *__restrict__ vp, const uint8_t *__restrict__ ip, uint32_t T,
+                                         uint32_t nseg, uint32_t before, const double *__restrict__ x, const Acc &acc,
+                                         const WaveLds &L, int lane_)
+{
+    const int lane = opaque_v(lane_);
+    // 256 entries from q on; TAIL: fewer
+    auto quads = [&](uint32_t q, auto tail_tag) __attribute__((always_inline)) {
+        constexpr bool TAIL = decltype(tail_tag)::value;
+        const uint32_t t = q + 4u * (uint32_t)lane;
+        double v[4], xv[4], p[4];
+        uint8_t id[4];
+        if constexpr (TAIL) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t j = min(t + (uint32_t)i, T - 1u);
+                v[i] = vp[j];
+                id[i] = ip[j];
+            }
+        } else {
+            __builtin_memcpy(v, vp + t, sizeof(v));
+            __builtin_memcpy(id, ip + t, sizeof(id));
+        }
+        // end bits: of the lane's entries, of the next lane's (none for the
+        // last of 16 lanes), of the entry before
+        const uint64_t word = L.ends[q / kWave + (uint32_t)(lane >> 4)];
+        const int sh = 4 * (lane & 15);
+        const uint32_t nib = (uint32_t)(word >> sh) & 15u, next = (uint32_t)(word >> sh) >> 4 & 15u;
+        const bool taken = sh && nib && !((word >> ((sh - 1) & 63)) & 1ull);
+        const uint32_t cnt = (uint32_t)__popc(nib), incl = wave_incl_scan_dpp(cnt);
+        const uint32_t own0 = before + incl - cnt;
+        before += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        uint32_t r[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t own = own0 + (uint32_t)__popc(nib & ((1u << i) - 1u));
+            if (TAIL) own = min(own, nseg - 1u);
+            r[i] = L.to[own];
+            xv[i] = x[L.bc[own] + (uint32_t)id[i]];
+            if (TAIL && t + (uint32_t)i >= T) {
+                v[i] = 0.0;
+                xv[i] = 0.0;
+            }
+        }
+        p[0] = v[0] * xv[0];
+#pragma unroll
+        for (int i = 1; i < 4; i++) p[i] = __builtin_fma(v[i], xv[i], (nib >> (i - 1)) & 1u ? 0.0 : p[i - 1]);
+        const uint32_t last = TAIL ? (t < T ? min(T - t, 4u) - 1u : 4u) : 3u;  // (4: no entries)
+        const bool open = last < 4u && !((nib >> last) & 1u);
+        const double in = dpp_f64<DPP_ROW_SHL1>(nib & 1u ? p[0] : nib & 2u ? p[1] : nib & 4u ? p[2] : p[3]);
+        if (open && next) p[3] += in;
+        uint32_t put = taken ? nib & (nib - 1u) : nib;
+        if (open) put |= 8u;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if ((put >> i) & 1u) atomicAdd(&acc.hi[r[i]], p[i]);
+    };
+    uint32_t q = 0;
+#pragma unroll 1
+    for (; q + (uint32_t)(4 * kWave) <= T; q += (uint32_t)(4 * kWave)) quads(q, std::false_type{});
+    const uint32_t left = T - q;
+    if (left > (uint32_t)kWave) {
+        quads(q, std::true_type{});
+    } else if (left) {  // one entry per lane, each added to the strip's sums
+        const uint32_t t = q + min((uint32_t)lane, left - 1u);
+        const double v = vp[t];
+        const uint32_t id = ip[t];
+        const uint64_t m = L.ends[q / kWave];
+        const uint32_t own = min((uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, before)),
+                                 nseg - 1u);
+        const uint32_t r = L.to[own];
+        const double xv = x[L.bc[own] + id];
+        if ((uint32_t)lane < left) atomicAdd(&acc.hi[r], v * xv);
+    }
+}
+
 // CSR group, blocks [b0, b1) whose first value is at offset e.  Chunks of 256
 // block rows (256 / s blocks), four consecutive rows of a block per lane: the
 // rows that hold entries are the chunk's segments (their number in L.to, the
 // block's first column in L.bc), the row pointers give their ends, and the
-// entries are taken as in the COO walk.
+// entries are taken in storage order (csr_sums; FP32 values as COO blocks).
 // Bound: memory latency.  When the lane of a row walked the row's entries by
 // itself, one load of 3-entry rows touched 12 lines instead of 4 and waited
 // for the row pointers, and a long row held up the wave for its whole length
@@ -444,8 +529,11 @@ __device__ __forceinline__ void csr_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
             }
             if (w) before = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan_dpp(before), kWave - 1);
             wave_sync();
-            seg_windows<VT, uint8_t, COMP, SEG_CSR, 4>(val + (e + w), ccol + (e + w), Tw, nseg, before, k, x, acc, L,
-                                                       lane);
+            if constexpr (COMP)
+                seg_windows<VT, uint8_t, COMP, SEG_CSR, 4>(val + (e + w), ccol + (e + w), Tw, nseg, before, k, x, acc,
+                                                           L, lane);
+            else
+                csr_sums(val + (e + w), ccol + (e + w), Tw, nseg, before, x, acc, L, lane);
             wave_sync();
         }
         e += T;
