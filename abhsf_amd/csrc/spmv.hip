@@ -1113,8 +1113,16 @@ struct StripArgs {
     double alpha, beta;
 };
 
+// Waves per SIMD at least (registers): FP32 values at s <= 16 wait on memory
+// and took 81 registers, five waves (27-point stencil 160^3 s = 16 tiled 1440
+// us, six 1257; banded n = 10^6 bandwidth 10 s = 8 107 -> 90; R-MAT scale 20
+// s = 16 tiled pays 115 -> 121).  At s >= 32 a sixth wave costs more than it
+// gives (2e6 uniform random columns, 24 a row, s = 64 tiled 413 -> 464).
+template <typename IT, bool COMP>
+constexpr int strip_min_waves() { return COMP && sizeof(IT) == 1 ? 6 : 1; }
+
 template <typename VT, typename BT, typename IT, typename RT, bool COMP, bool TILED>
-__global__ __launch_bounds__(64 * kStripWaves) void k_spmv_strip(StripArgs)
+__global__ __launch_bounds__(64 * kStripWaves, (strip_min_waves<IT, COMP>())) void k_spmv_strip(StripArgs)
 {
     constexpr int kWaves = kStripWaves;
     // s rows, or a tile's (kTileRows; kTileRowsComp compensated, lo half at +256)
