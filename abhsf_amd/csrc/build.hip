@@ -285,7 +285,7 @@ __global__ void k_emit(const uint32_t *__restrict__ flag, const uint32_t *__rest
 
 // Tiled COO order, step 1: sort key of every COO block b = (group of its
 // strip, block column, strip within the group).  Groups are consecutive strip
-// ranges numbered in strip order (a tile, or one strip), so sorting by the
+// ranges numbered in strip order (a tile, a group, or one strip), so sorting by the
 // key reorders blocks only inside tiles.  The strip of b is the last I with
 // sptr[I] <= b (empty strips share their start with the next strip).
 __global__ void k_tile_keys(const uint32_t *__restrict__ sptr, int64_t M, uint64_t nb, const void *__restrict__ bcol,
@@ -694,7 +694,7 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
             int64_t acc = 0;
             for (uint32_t b = b0; b < b1; b++) {
                 const int64_t wz = work(x, b);
-                const int p = panels > 1 ? panel_of[bc[x][b]] : 0;
+                const int p = panel_of[bc[x][b]];
                 if (b > ub && (p != up || acc + wz > unit)) {
                     units.insert(units.end(), {(uint32_t)x | ((uint32_t)I << 2), ub, b, (uint32_t)ue});
                     unit_panel.push_back((uint8_t)up);

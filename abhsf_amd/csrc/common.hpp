@@ -83,17 +83,6 @@ __device__ inline void wave_sync()
 
 __device__ inline int lane_id() { return __lane_id(); }
 
-__device__ inline uint32_t wave_incl_scan_u32(uint32_t v)
-{
-    const int lane = lane_id();
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        uint32_t t = __shfl_up(v, o, kWave);
-        if (lane >= o) v += t;
-    }
-    return v;
-}
-
 template <int G>
 __device__ inline double group_sum(double v)
 {

@@ -128,7 +128,7 @@ __device__ inline void acc_add(double &hi, double &lo, double v, double xv)
     }
 }
 
-// Sum (hi, lo) over aligned groups of P lanes (P in {1, 2, 4, 8}).
+// Sum (hi, lo) over aligned groups of P lanes (P = 2 or 4).
 template <bool COMP, int P>
 __device__ inline void group_reduce_p(double &hi, double &lo)
 {
@@ -143,9 +143,8 @@ __device__ inline void group_reduce_p(double &hi, double &lo)
             hi = s;
             lo += tl + e;
         };
-        if constexpr (P >= 2) step(std::integral_constant<int, DPP_QUAD_XOR1>{});
-        if constexpr (P >= 4) step(std::integral_constant<int, DPP_QUAD_XOR2>{});
-        if constexpr (P >= 8) step(std::integral_constant<int, DPP_ROW_HALF_MIRROR>{});
+        step(std::integral_constant<int, DPP_QUAD_XOR1>{});
+        if constexpr (P == 4) step(std::integral_constant<int, DPP_QUAD_XOR2>{});
     }
 }
 
@@ -172,15 +171,12 @@ __device__ __forceinline__ void row_reduce(int k, double &hi, double &lo)
     if (k > 3) step(std::integral_constant<int, DPP_ROW_MIRROR>{});
 }
 
+// (P = 1, 2 or 4)
 template <bool COMP>
 __device__ inline void group_reduce(int P, double &hi, double &lo)
 {
-    switch (P) {
-    case 1: break;
-    case 2: group_reduce_p<COMP, 2>(hi, lo); break;
-    case 4: group_reduce_p<COMP, 4>(hi, lo); break;
-    default: group_reduce_p<COMP, 8>(hi, lo); break;
-    }
+    if (P == 2) group_reduce_p<COMP, 2>(hi, lo);
+    else if (P == 4) group_reduce_p<COMP, 4>(hi, lo);
 }
 
 // LDS of one wave besides its accumulator: a chunk's segments (COO blocks, or
@@ -667,8 +663,8 @@ __device__ __forceinline__ void coo_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint
     }
 }
 
-// Bitmap or dense group of strip I.  Each lane owns cw consecutive row-major
-// positions of the block (P = s / cw lanes per row); it accumulates its
+// Bitmap or dense group of a strip, s >= 16.  Each lane owns cw consecutive
+// row-major positions of the block (P = s / cw lanes per row); it accumulates its
 // products in registers, the P lanes of a row are summed with DPP, and the
 // first lane of the row adds the sum to the strip accumulator.
 template <typename VT, typename BT, bool COMP>
@@ -680,8 +676,8 @@ __device__ __forceinline__ void bmdn_r1(MatPtr A_, int sc, uint32_t b0, uint32_t
     const int lane = opaque_v(lane_);
     const int s = A->s, k = A->k;
     const uint32_t ss = (uint32_t)s * (uint32_t)s;
-    const uint32_t cw = s >= 64 ? (uint32_t)s : (ss >= 64 ? ss / 64 : 1u);
-    const int npass = (int)((ss + 64u * cw - 1) / (64u * cw));
+    const uint32_t cw = s >= 64 ? (uint32_t)s : ss / 64u;
+    const int npass = (int)(ss / (64u * cw));
     const int P = (int)((uint32_t)s / cw);
     const int64_t n = A->n;
     const VT *__restrict__ val = glob<VT>(A->val[sc]);
@@ -693,36 +689,33 @@ __device__ __forceinline__ void bmdn_r1(MatPtr A_, int sc, uint32_t b0, uint32_t
 #pragma unroll 1
         for (int q = 0; q < npass; q++) {
             const uint32_t pbase = ((uint32_t)q * 64u + (uint32_t)lane) * cw;
-            const bool valid = pbase < ss;
             const uint32_t row = pbase >> k, col0 = pbase & ((uint32_t)s - 1);
             const int64_t gc0 = c0 + col0;
             double hi = 0.0, lo = 0.0;
             if (sc == DENSE) {
-                if (valid) {
-                    const VT *vp = val + db + pbase;
-                    // double2 loads of x need a 16-byte aligned x (a caller may pass
-                    // x + 1 of an array): otherwise the scalar walk below
-                    if (gc0 + (int64_t)cw <= n && (cw & 1) == 0 && x_aligned16(x)) {
+                const VT *vp = val + db + pbase;
+                // double2 loads of x need a 16-byte aligned x (a caller may pass
+                // x + 1 of an array): otherwise the scalar walk below
+                if (gc0 + (int64_t)cw <= n && (cw & 1) == 0 && x_aligned16(x)) {
 #pragma unroll 4
-                        for (uint32_t c = 0; c < cw; c += 2) {
-                            const double2 xv = *reinterpret_cast<const double2 *>(x + gc0 + c);
-                            double v0, v1;
-                            if constexpr (sizeof(VT) == 8) {
-                                const double2 vv = *reinterpret_cast<const double2 *>(vp + c);
-                                v0 = vv.x;
-                                v1 = vv.y;
-                            } else {
-                                const float2 vv = *reinterpret_cast<const float2 *>(vp + c);
-                                v0 = vv.x;
-                                v1 = vv.y;
-                            }
-                            acc_add<COMP>(hi, lo, v0, xv.x);
-                            acc_add<COMP>(hi, lo, v1, xv.y);
+                    for (uint32_t c = 0; c < cw; c += 2) {
+                        const double2 xv = *reinterpret_cast<const double2 *>(x + gc0 + c);
+                        double v0, v1;
+                        if constexpr (sizeof(VT) == 8) {
+                            const double2 vv = *reinterpret_cast<const double2 *>(vp + c);
+                            v0 = vv.x;
+                            v1 = vv.y;
+                        } else {
+                            const float2 vv = *reinterpret_cast<const float2 *>(vp + c);
+                            v0 = vv.x;
+                            v1 = vv.y;
                         }
-                    } else {
-                        for (uint32_t c = 0; c < cw; c++)
-                            if (gc0 + c < n) acc_add<COMP>(hi, lo, (double)vp[c], x[gc0 + c]);
+                        acc_add<COMP>(hi, lo, v0, xv.x);
+                        acc_add<COMP>(hi, lo, v1, xv.y);
                     }
+                } else {
+                    for (uint32_t c = 0; c < cw; c++)
+                        if (gc0 + c < n) acc_add<COMP>(hi, lo, (double)vp[c], x[gc0 + c]);
                 }
             } else {
                 // bitmap: popcount of my positions -> value offset by a wave scan
@@ -730,45 +723,42 @@ __device__ __forceinline__ void bmdn_r1(MatPtr A_, int sc, uint32_t b0, uint32_t
                 const uint32_t w0 = pbase >> 6, sh = pbase & 63;
                 const uint64_t m = cw >= 64 ? ~0ull : ((1ull << cw) - 1ull);
                 uint32_t cnt = 0;
-                if (valid)
-                    for (uint32_t w = 0; w < nw; w++) cnt += __popcll((words[w0 + w] >> sh) & m);
+                for (uint32_t w = 0; w < nw; w++) cnt += __popcll((words[w0 + w] >> sh) & m);
                 const uint32_t incl = wave_incl_scan_dpp(cnt);
                 const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
                 uint64_t off = vb + incl - cnt;
-                if (valid) {
-                    for (uint32_t w = 0; w < nw; w++) {
-                        uint64_t bits = (words[w0 + w] >> sh) & m;
-                        const int64_t xb = gc0 + (int64_t)w * 64;
-                        // four set bits per step so their loads are in flight together
-                        while (bits) {
-                            const uint32_t c0 = (uint32_t)__builtin_ctzll(bits);
-                            bits &= bits - 1;
-                            const bool h1 = bits != 0;
-                            const uint32_t c1 = h1 ? (uint32_t)__builtin_ctzll(bits) : c0;
-                            bits &= bits - 1;
-                            const bool h2 = bits != 0;
-                            const uint32_t c2 = h2 ? (uint32_t)__builtin_ctzll(bits) : c0;
-                            bits &= bits - 1;
-                            const bool h3 = bits != 0;
-                            const uint32_t c3 = h3 ? (uint32_t)__builtin_ctzll(bits) : c0;
-                            bits &= bits - 1;
-                            const double v0 = (double)val[off];
-                            const double v1 = (double)val[h1 ? off + 1 : off];
-                            const double v2 = (double)val[h2 ? off + 2 : off];
-                            const double v3 = (double)val[h3 ? off + 3 : off];
-                            const double x0 = x[xb + c0], x1 = x[xb + c1], x2 = x[xb + c2], x3 = x[xb + c3];
-                            acc_add<COMP>(hi, lo, v0, x0);
-                            if (h1) acc_add<COMP>(hi, lo, v1, x1);
-                            if (h2) acc_add<COMP>(hi, lo, v2, x2);
-                            if (h3) acc_add<COMP>(hi, lo, v3, x3);
-                            off += 1u + h1 + h2 + h3;
-                        }
+                for (uint32_t w = 0; w < nw; w++) {
+                    uint64_t bits = (words[w0 + w] >> sh) & m;
+                    const int64_t xb = gc0 + (int64_t)w * 64;
+                    // four set bits per step so their loads are in flight together
+                    while (bits) {
+                        const uint32_t c0 = (uint32_t)__builtin_ctzll(bits);
+                        bits &= bits - 1;
+                        const bool h1 = bits != 0;
+                        const uint32_t c1 = h1 ? (uint32_t)__builtin_ctzll(bits) : c0;
+                        bits &= bits - 1;
+                        const bool h2 = bits != 0;
+                        const uint32_t c2 = h2 ? (uint32_t)__builtin_ctzll(bits) : c0;
+                        bits &= bits - 1;
+                        const bool h3 = bits != 0;
+                        const uint32_t c3 = h3 ? (uint32_t)__builtin_ctzll(bits) : c0;
+                        bits &= bits - 1;
+                        const double v0 = (double)val[off];
+                        const double v1 = (double)val[h1 ? off + 1 : off];
+                        const double v2 = (double)val[h2 ? off + 2 : off];
+                        const double v3 = (double)val[h3 ? off + 3 : off];
+                        const double x0 = x[xb + c0], x1 = x[xb + c1], x2 = x[xb + c2], x3 = x[xb + c3];
+                        acc_add<COMP>(hi, lo, v0, x0);
+                        if (h1) acc_add<COMP>(hi, lo, v1, x1);
+                        if (h2) acc_add<COMP>(hi, lo, v2, x2);
+                        if (h3) acc_add<COMP>(hi, lo, v3, x3);
+                        off += 1u + h1 + h2 + h3;
                     }
                 }
                 vb += tot;
             }
             group_reduce<COMP>(P, hi, lo);
-            if (valid && (lane & (P - 1)) == 0) {
+            if ((lane & (P - 1)) == 0) {
                 if constexpr (COMP) {
                     double s2, e2;
                     two_sum(acc.hi[row], hi, s2, e2);
@@ -956,11 +946,6 @@ __device__ __forceinline__ void bitmap_r1(MatPtr A, uint32_t b0, uint32_t b1, ui
     else bmdn_r1<VT, BT, COMP>(A, BITMAP, b0, b1, e, x, acc, lane);
 }
 
-// Work items: items [0, n_light) are light items -- whole strips light[p] for
-// p in [pack[item], pack[item + 1]) (p = item without pack; strip p without
-// light) -- whose rows are written to y; items n_light + u are
-// units u of heavy strips: one scheme group's block range, whose partial sums
-// go to part[u] and are combined by k_spmv_fixup.
 // Workgroups are dispatched to the 8 XCDs round-robin.  Renumber them so that
 // each XCD (and its L2) receives runs of kRun consecutive work items (the x
 // windows of neighbouring strips stay in one L2) while the runs rotate over
@@ -978,6 +963,11 @@ __device__ inline int64_t xcd_block_id()
 
 // One work item of one matrix (see Balance): the wave accumulates in acc_buf
 // (s doubles, 2s when compensated) and writes y rows or a unit's partials.
+// Work items: items [0, n_light) are light items -- whole strips light[p] for
+// p in [pack[item], pack[item + 1]) (p = item without pack; strip p without
+// light) -- whose rows are written to y; items n_light + u are
+// units u of heavy strips: one scheme group's block range, whose partial sums
+// go to part[u] and are combined by k_spmv_fixup.
 // TL: 0 the matrix is not tiled, 1 it is, 2 either (read from B.tiled); the
 // single-matrix kernels are compiled for 0 or 1 so that each carries only one
 // of the light-item paths (scalar-register pressure).
@@ -1100,11 +1090,6 @@ __device__ __forceinline__ void spmv_item(MatPtr A, BalPtr B, int64_t item, cons
     wave_sync();  // the next item reuses the LDS buffers
 }
 
-// Work items: items [0, n_light) are light items -- whole strips light[p] for
-// p in [pack[item], pack[item + 1]) (p = item without pack; strip p without
-// light) -- whose rows are written to y; items n_light + u are
-// units u of heavy strips: one scheme group's block range, whose partial sums
-// go to part[u] and are combined by k_spmv_fixup.
 struct StripArgs {
     DevMat A;
     Balance B;
