@@ -785,12 +785,19 @@ void Storage::build_balance(int64_t unit, hipStream_t st, int panels, int tile_r
     std::vector<uint32_t> grank, gtpos, coo_rng;
     uint64_t nrank = 0;
     int64_t ntiles = 0;  // tiles of several strips (the first items)
-    // strips the kernel takes in groups: any up to s = 8; at s = 16 few-entry
-    // bitmap blocks (position by position in a group), from 32 on COO and CSR
-    // blocks only (its other paths take a strip at a time)
+    // strips the kernel takes in groups: any up to s = 8; from 32 on COO and CSR
+    // blocks only (its other paths take a strip at a time).  At s = 16 a group's
+    // bitmap blocks go position by position, which is more work than the lane
+    // walk (27-point stencil 100^3, 432 entries a strip, 214 us alone, 268 and
+    // more in groups): strips of few entries, and only where there are many
+    // strips.  us alone / in groups, FP64 (FP32 values):
+    //   Laplacian 500^2  (15 625 strips) 15.9 / 18.3 (17.2 / 26.6)   2e5 rows, four 8-row blocks each  14.9 / 18.7
+    //   Laplacian 1000^2 (62 500)          66 / 51   (76 / 76)       1e6 rows, two 8-row blocks each   62 / 51 (72 / 76)
+    //   Laplacian 1500^2 (140 625)        140 / 96   (161 / 148)     3e6 rows, two 8-row blocks each  171 / 109 (202 / 173)
+    const int64_t bm16 = val_bytes == 4 ? 1 << 17 : 3 << 14;
     auto groupable = [&](uint32_t I) {
         const bool bm = ep[BITMAP][I + 1] != ep[BITMAP][I], dn = ep[DENSE][I + 1] != ep[DENSE][I];
-        return s <= 8 || (!dn && (!bm || (s == 16 && strip_work(I) <= 128)));
+        return s <= 8 || (!dn && (!bm || (s == 16 && M >= bm16 && strip_work(I) <= 128)));
     };
     if (tile_rows > 0) {
         // items: tiles of light strips whose entries are all COO (or none), up
