@@ -350,7 +350,12 @@ __global__ void k_tile_move(uint64_t nb, const uint32_t *__restrict__ perm, cons
 // Units of heavy strip groups: workgroup g takes the blocks [b0, b1) of range
 // g = {scheme | strip << 2, b0, b1, first value} and starts a unit at every
 // block whose first value lies in another multiple of `unit` entries (counted
-// from the range's start) than the block's before it.  out null: counts[g] =
+// from the range's start) than the block's before it, and at every block of
+// unit / 2 entries or more that reaches into the next one: no unit holds more
+// than 3/2 `unit` unless it is one block (27-point stencil 40^3 s = 256, 250
+// strips: units of two such blocks 15.3 us, now 12.4; FP32 values 19.1, 16.0.
+// The line at unit / 4 12.0 and 15.1, but more units: R-MAT scale 20 s = 256
+// tiled, FP32 values, 107.7 -> 109.7).  out null: counts[g] =
 // number of units; else the units go to out[4 * counts[g] ..] (counts then
 // holds the first unit of every range).  dense: blocks of ss positions each.
 __global__ __launch_bounds__(kT) void k_units(const uint32_t *__restrict__ ranges, Four<const uint16_t *> z1,
@@ -383,7 +388,8 @@ __global__ __launch_bounds__(kT) void k_units(const uint32_t *__restrict__ range
             else if (wave == 0) wp = prev;
             else wp = ok ? (x == DENSE ? ss : (uint32_t)z1.p[x][i - 1] + 1u) : 0u;
         }
-        const bool start = ok && (i == b0 || at / unit != (at - wp) / unit);
+        const bool start = ok && (i == b0 || at / unit != (at - wp) / unit ||
+                                  (w >= unit / 2u && at / unit != (at + w - 1u) / unit));
         const uint64_t m = __ballot(start);
         if (lane == 0) wsum[1][wave] = (uint32_t)__popcll(m);
         __syncthreads();

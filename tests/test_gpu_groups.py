@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from abhsf_amd import AbhsfMatrix, synth
-from test_gpu_segments import CASES, check, with_integers
+from test_gpu_segments import CASES, check, strip_of_blocks, with_integers
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +46,20 @@ def test_chunk_edge_matrices_hold_their_blocks(gpu, name):
     print(f"case blocks {name} {blocks}", flush=True)
     own = name.split("_")[0]
     assert blocks == {"coo": 2, "csr": 0, "bitmap": 0, "dense": 0, **{own: first + (2 if own == "coo" else 0)}}
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("counts,units", [
+    ([1500] * 4, 4),               # two do not fit 2048 entries
+    ([2048] * 3, 3), ([2049, 2047, 600], 3),
+    ([7000], 1),                   # one block is never cut
+    ([1100] * 6, 6),               # the even ones reach into the next multiple, the odd ones begin there
+    ([1020] * 6, 3), ([300] * 20, 3),  # blocks below 1024 entries stay with the unit they begin in
+])
+def test_units_of_a_heavy_strip(gpu, counts, units, precision):
+    """CSR blocks of one heavy strip: how many units it is cut into, and the
+    exact product."""
+    A = strip_of_blocks(256, counts, 1, 3)
+    print(f"case units {counts} {precision}", flush=True)
+    st = check(A, 256, "balanced", precision)
+    assert st["work_items"] == units + 1  # (the ragged second strip)
