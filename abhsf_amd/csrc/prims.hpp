@@ -61,8 +61,8 @@ class DevBuf {
 };
 
 // Device scratch of one operation on a stream, handed out piece by piece.  A
-// conversion needs some thirty pieces, about 36 bytes an entry in all, and
-// allocating and freeing them every time cost more than its kernels: a free
+// conversion needs some thirty pieces (24 bytes an entry and 45 a block, and
+// the sort's 12.5 an entry, which are idle after it), and allocating and freeing them every time cost more than its kernels: a free
 // waits for the device, and freed memory is cleared before it is given out
 // again (converting R-MAT scale 20, 0.9 GB of scratch, again and again: 12 ms
 // at first, 28 ms once the clearing lags behind).  Small pieces share chunks;

@@ -40,7 +40,7 @@ namespace {
 // each group starts from a pointer and a lane number the compiler cannot see
 // through.  With the descriptor passed by value the compiler kept fields and
 // lane addresses of all four groups for the whole kernel: 83 VGPRs and 57
-// spilled SGPRs where the same groups now take 61 and 3.
+// spilled SGPRs where the same groups now take 67 and none (FP64 values).
 using MatPtr = const __attribute__((address_space(4))) DevMat *;
 using BalPtr = const __attribute__((address_space(4))) Balance *;
 
@@ -457,8 +457,8 @@ __device__ __forceinline__ void csr_sums(const double *__restrict__ vp, const ui
 // Bound: memory latency.  When the lane of a row walked the row's entries by
 // itself, one load of 3-entry rows touched 12 lines instead of 4 and waited
 // for the row pointers, and a long row held up the wave for its whole length
-// (R-MAT scale 20 s = 256 tiled, 10 % of the entries in CSR blocks, 128 -> 64
-// us; block_mix n = 2^22 s = 128 tiled 990 -> 686 us).
+// (R-MAT scale 20 s = 256 tiled, 10 % of the entries in CSR blocks, 124 -> 69
+// us; block_mix n = 2^22 s = 128 tiled 983 -> 654 us).
 // A group of T > 1 strips from I0 on: strip I0 + t has the accumulator rows
 // from t << k on.
 template <typename VT, typename BT, typename RT, bool COMP>
@@ -586,9 +586,9 @@ __device__ __forceinline__ void group_rows(uint32_t first, uint32_t cb, uint32_t
 // Bound: memory latency and the x gathers.  Before, a binary search of the
 // prefix sums located every entry beyond a block's first two, which the
 // block's lane took by itself: 62 VALU instructions per 64 entries (28 now)
-// and loads that waited for the metadata.  With the CSR walk above: 27-point
-// stencil 160^3 s = 64 396 -> 262 us (4.4 TB/s), R-MAT scale 22 s = 256 tiled
-// 470 -> 354 us, scale 20 s = 64 210 -> 168 us.
+// and loads that waited for the metadata.  Together with entries in storage
+// order for CSR blocks: 27-point stencil 160^3 s = 64 394 -> 249 us (4.7 TB/s),
+// R-MAT scale 22 s = 256 tiled 470 -> 356 us.
 enum CooMode { COO_STRIP, COO_TILE, COO_GROUP };
 
 template <typename VT, typename BT, typename IT, bool COMP, int MODE = COO_STRIP>
@@ -780,8 +780,8 @@ __device__ __forceinline__ void bmdn_r1(MatPtr A_, int sc, uint32_t b0, uint32_t
 // strip accumulator.  Block columns and, in a group of T > 1 strips from I0 on,
 // the strips' rows come from LDS, 256 blocks at a time.
 // Bound: memory latency.  One block per step, as before, was two round trips
-// per block: 2048^2 Laplacian s = 8 (a bitmap block per strip) 787 -> 118 us
-// with groups of strips, banded n = 10^6 bandwidth 40 s = 8 422 -> 186 us.
+// per block: 2048^2 Laplacian s = 8 (a bitmap block per strip) 786 -> 114 us
+// with groups of strips, banded n = 10^6 bandwidth 10 s = 8 220 -> 58 us.
 template <typename VT, typename BT, bool COMP, int SC>
 __device__ __forceinline__ void small_r1(MatPtr A_, uint32_t b0, uint32_t b1, uint32_t e, const double *__restrict__ x,
                                          const Acc &acc, WaveLds &L, int lane_, int64_t I0, int T_)

@@ -63,11 +63,12 @@ constexpr int64_t kTileWork = ABHSF_TILE_WORK;  // entries per tile at most
 // twice as many strips is not grouped, its waves fill the chip by themselves).
 // A wave needs about 4 us for a strip of any small size (a chain of memory
 // round trips), so strips taken one by one, or several in turn in one wave,
-// cost their number: 2048^2 Laplacian s = 32 (160 entries a strip) 239 -> 64
-// us, s = 8 787 -> 118 us, R-MAT scale 20 s = 64 211 -> 78 us, a batch of 100
-// matrices s = 32 530 -> 289 us.  At 1024 / 4096 / 16384 items: batch 277 / 306
-// / 302 us, 100 000 rows of random 8-row blocks s = 32 8.8 / 8.1 / 8.3 us (8.2
-// here), the others alike.
+// cost their number.  With the segment walks, repeated calls on one x: 2048^2
+// Laplacian s = 32 (160 entries a strip) 243 -> 61 us, s = 8 786 -> 114 us,
+// R-MAT scale 20 s = 64 204 -> 76 us (among other calls 237 -> 104), a batch of
+// 100 matrices s = 32 530 -> 289 us when called alone.  At 1024 / 4096 / 16384
+// items: batch 277 / 306 / 302 us, 100 000 rows of random 8-row blocks s = 32
+// 8.8 / 8.1 / 8.3 us (8.2 here), the others alike.
 constexpr int kGroupRows = 256;
 constexpr int64_t kGroupWork = 2048;
 constexpr int64_t kGroupItems = 2048;
